@@ -72,8 +72,9 @@ def draw(rng):
         n = rng.choice([4, 8])
         return dict(kind=kind, n=n, paths=_log_int(rng, 5, 3**n), via=rng.choice(["host", "device", "graph"]))
     if kind == "param10":
-        paths = _log_int(rng, 30, 200000)
-        return dict(kind=kind, targets=-(-paths // 1024), paths=paths, learned=rng.random() < 0.5,
+        plain = rng.random() < 0.5  # the plain rule takes about twice the learned rule's time
+        paths = _log_int(rng, 30, 110000 if plain else 230000)
+        return dict(kind=kind, targets=-(-paths // 1024), paths=paths, learned=not plain,
                     via=rng.choice(["host", "device", "graph"]))
     if kind == "mixed":
         plain = rng.random() < 0.5
