@@ -887,10 +887,14 @@ bool generate_multi_source(const hcg_homotopy_desc* const* hs, int nsys, std::st
     int phase = 0, k = -1, s = 0;
     while (true) {
         int ended = 0;
-        const unsigned long long fetch = wave_refill_mask(phase == 0, refill);
-        if (phase == 0) {
+        const unsigned long long fetch = wave_refill_mask(phase != 1, refill);
+        if (phase != 1) {
             if (!fetch) continue;
-            int kg = wave_fetch(fetch, m.next_path);
+            const int kg = wave_fetch(fetch, m.next_path);
+            if (phase == 2) {
+)" << each("@NS::lane_close(@L, @A, k, T);")
+       << R"(            }
+            phase = 0;
             if (kg >= m.total) break;
             s = 0;
             while (s + 1 < m.nsys && kg >= m.offset[s + 1]) s++;
@@ -902,10 +906,7 @@ bool generate_multi_source(const hcg_homotopy_desc* const* hs, int nsys, std::st
         } else {
 )" << each("{ @NS::lane_iter(@L); ended = @NS::lane_ended(@L); }")
        << R"(        }
-        if (ended) {
-)" << each("@NS::lane_finish(@L, @A, k, T);")
-       << R"(            phase = 0;
-        }
+        if (ended) phase = 2;
     }
     atomicAdd(&m.sys[0].counters[0], (unsigned long long)T.steps);
     atomicAdd(&m.sys[0].counters[1], (unsigned long long)T.newton);

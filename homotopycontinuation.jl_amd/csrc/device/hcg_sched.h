@@ -1,10 +1,11 @@
 // Work distribution of the persistent tracker kernels over the lanes of a wave.
 //
-// A lane whose path has ended does not start its next path at once: starting a path
-// (tracker and predictor initialization, a condition estimate) costs a few tracker steps,
-// and while one lane does it the other 63 lanes of the wave wait.  Idle lanes therefore
-// wait until at least `refill` of the wave's live lanes are idle (or all of them are),
-// then take their next paths from the work queue together, with one atomic per wave.
+// A lane whose path has ended does not close it and start its next path at once: closing a
+// path (refinement in double-double, a condition estimate, the record) and starting one
+// (tracker and predictor initialization) cost a few tracker steps each, and while one lane
+// does it the other 63 lanes of the wave wait.  Idle lanes therefore wait until at least
+// `refill` of the wave's live lanes are idle (or all of them are), then close their paths and
+// take their next ones from the work queue together, with one atomic per wave.
 #pragma once
 #include "hcgpu_types.h"
 

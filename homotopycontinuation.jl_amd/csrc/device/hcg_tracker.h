@@ -3,8 +3,8 @@
 // Compiled by hipRTC together with the generated system functions of one homotopy
 // (HCG_N, HCG_KIND, sysG_* / sysF_*).  Each lane repeatedly takes a path index from a
 // device work queue (atomic counter), tracks it with one tracker step per loop
-// iteration, and writes its PathResult record when the path ends; finished lanes of a
-// wave take their next paths together (hcg_sched.h).
+// iteration; finished lanes of a wave write their PathResult records and take their next
+// paths together (hcg_sched.h).
 //
 // Algorithm (restated from the reference, same arithmetic contract as the oracle):
 //   tracker            src/tracker.jl:517-996     predictor  src/predictor.jl:124-371
@@ -26,23 +26,23 @@ extern "C" __global__ void __launch_bounds__(64, HCG_WAVES_PER_EU) hcg_track_ker
     lane_setup(L, a, mw);
     LaneTotals T = {0, 0, 0, 0.0};
     const int refill = refill_threshold(a.opts);
-    int phase = 0;  // 0: idle, 1: tracking
+    int phase = 0;  // 0: idle, 1: tracking, 2: path k has ended and is not closed yet
     int k = -1;
     while (true) {
-        const unsigned long long fetch = wave_refill_mask(phase == 0, refill);
-        if (phase == 0) {
+        const unsigned long long fetch = wave_refill_mask(phase != 1, refill);
+        if (phase != 1) {
             if (!fetch) continue;  // wait for more idle lanes of this wave
-            k = wave_fetch(fetch, a.next_path);
+            const int kn = wave_fetch(fetch, a.next_path);
+            if (phase == 2) lane_close(L, a, k, T);
+            phase = 0;
+            k = kn;
             if (k >= a.npaths) break;
             if (!lane_begin(L, a, k)) continue;
             phase = 1;
         } else {
             lane_iter(L);
         }
-        if (lane_ended(L)) {
-            lane_finish(L, a, k, T);
-            phase = 0;
-        }
+        if (lane_ended(L)) phase = 2;
     }
     atomicAdd(&a.counters[0], (unsigned long long)T.steps);
     atomicAdd(&a.counters[1], (unsigned long long)T.newton);

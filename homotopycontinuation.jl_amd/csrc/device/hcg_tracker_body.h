@@ -24,6 +24,12 @@ enum { NEWT_CONVERGED = 0, NEWT_TERMINATED, NEWT_MAX_ITERS, NEWT_SINGULARITY };
 #define FL_MIXED (80.0 * NN * NN + 26.0 * NN + FL_SOLVE)
 #define FL_FIXED (8.0 * NN * NN + 4.0 * NN + FL_SOLVE)
 
+struct NewtRes { int code; double accuracy; int iters; double omega, theta, mu_low, norm_dx0; };
+
+// End-of-path work left for lane_close: the rest of the step that reached the end of the
+// segment (PEND_STEP), then tracking_stopped! (PEND_STOP).
+enum { PEND_NONE = 0, PEND_STEP, PEND_STOP };
+
 struct Lane {
     const hcg_options* o;
     // ParameterHomotopy data
@@ -81,6 +87,10 @@ struct Lane {
     const unsigned short* mlp_w;  // BF16 weights in LDS, or null (plain rule only)
     double flops;  // counted FP64 flops of this path
     int guard;     // loop iterations of the current path (each performs >= 1 tracker step)
+    // work at the end of a path that waits for the wave's next refill (lane_close)
+    int pend;
+    double pend_ds0;
+    NewtRes pend_res;
     // step log
     float* log_records;
     int* log_count;
@@ -589,7 +599,6 @@ __device__ __noinline__ void wnorm_update(Lane& L, const cplx* x) {
 }
 
 // ----------------------------- Newton corrector -----------------------------
-struct NewtRes { int code; double accuracy; int iters; double omega, theta, mu_low, norm_dx0; };
 
 __device__ __forceinline__ NewtRes mkres(int code, double acc, int iters, double omega, double theta, double mu_low, double ndx0) {
     NewtRes R; R.code = code; R.accuracy = acc; R.iters = iters; R.omega = omega; R.theta = theta; R.mu_low = mu_low; R.norm_dx0 = ndx0;
@@ -1008,23 +1017,42 @@ __device__ __noinline__ void log_step(Lane& L, const NewtRes& res, int acc) {
     r[15] = (float)(isnan(L.ds_plain) ? hc_log(seg_ds(L)) : hc_log(L.ds_plain));
 }
 
-// step!(tracker), src/tracker.jl:851-926; returns !last_step_failed
+// step!(tracker), src/tracker.jl:851-926; returns !last_step_failed.  The step that ends the path
+// (outside the singular endgame) returns with L.pend = PEND_STEP after its Newton correction, and
+// the next call does the rest: refinement in double-double and the predictor's update, several
+// ordinary evaluations' work, which lane_close runs for all ended lanes of a wave at once.
 __device__ __noinline__ int tracker_step(Lane& L) {
     const hcg_options* o = L.o;
-    cplx t = seg_t(L), dt = seg_dt(L), t1 = seg_t1(L);
-    const double ds0 = seg_ds(L);
-    predict(L, t, dt);
-    wnorm_update(L, L.xh);
-    NewtRes res = newton(L, L.xh, t1, L.mu, L.omega, L.extended_prec, 0, L.accepted == 0);
-    if (res.code == NEWT_CONVERGED && L.last_learned) L.learned_accepted++;
+    NewtRes res;
+    double ds0;
+    if (L.pend == PEND_STEP) {
+        res = L.pend_res;
+        ds0 = L.pend_ds0;
+        L.pend = PEND_NONE;
+    } else {
+        cplx t = seg_t(L), dt = seg_dt(L), t1 = seg_t1(L);
+        ds0 = seg_ds(L);
+        predict(L, t, dt);
+        wnorm_update(L, L.xh);
+        res = newton(L, L.xh, t1, L.mu, L.omega, L.extended_prec, 0, L.accepted == 0);
+        if (res.code == NEWT_CONVERGED && L.last_learned) L.learned_accepted++;
+        if (res.code == NEWT_CONVERGED) {
+            for (int i = 0; i < NN; i++) L.x[i] = L.xb[i];
+            L.ds_prev = seg_ds(L);
+            L.seg_s = L.seg_s1;
+            L.accuracy = res.accuracy;
+            L.mu = jmax(res.accuracy, DEPS);
+            L.omega_prev = L.omega;
+            L.omega = jmax(jmax(res.omega, 0.5 * L.omega), 0.1);
+            if (!L.singular_endgame && seg_is_done(L)) {
+                L.pend = PEND_STEP;
+                L.pend_res = res;
+                L.pend_ds0 = ds0;
+                return 1;
+            }
+        }
+    }
     if (res.code == NEWT_CONVERGED) {
-        for (int i = 0; i < NN; i++) L.x[i] = L.xb[i];
-        L.ds_prev = seg_ds(L);
-        L.seg_s = L.seg_s1;
-        L.accuracy = res.accuracy;
-        L.mu = jmax(res.accuracy, DEPS);
-        L.omega_prev = L.omega;
-        L.omega = jmax(jmax(res.omega, 0.5 * L.omega), 0.1);
         update_precision(L, res.mu_low);
         if (seg_is_done(L) && o->extended_precision && L.accuracy > 1e-14) {
             L.accuracy = refine_current_solution(L, 1e-14, 3);
@@ -1320,7 +1348,7 @@ __device__ __noinline__ void singular_post(Lane& L, bool max_steps) {
     if (!max_steps) {
         if (L.code != TC_SUCCESS) {
             L.eg_code = tc_to_eg(L.code);
-            tracking_stopped(L);
+            L.pend = PEND_STOP;  // tracking_stopped!, in lane_close
             return;
         }
         val_update(L, lam * L.sing_t);
@@ -1362,7 +1390,7 @@ __device__ __noinline__ void singular_post(Lane& L, bool max_steps) {
 // inner `while is_tracking: step!` loop flattened to one tracker step per call
 __device__ __noinline__ void eg_step(Lane& L) {
     const hcg_options* o = L.o;
-    if (!(L.singular_endgame && L.sing_phase == 1)) {
+    if (L.pend != PEND_STEP && !(L.singular_endgame && L.sing_phase == 1)) {
         if (L.steps_eg >= o->max_endgame_steps) { L.eg_code = EG_MAX_STEPS; return; }
         if (ext_steps(L) - L.ext_steps_eg_start > o->max_endgame_extended_steps) {
             bool allfinite = true;
@@ -1398,8 +1426,9 @@ __device__ __noinline__ void eg_step(Lane& L) {
     cplx tp = seg_t1(L);
     int jump = tp.re == 0.0 && tp.im == 0.0;
     int ok = tracker_step(L);
+    if (L.pend == PEND_STEP) return;  // the path has reached its end: continued by lane_close
     L.eg_code = tc_to_eg(L.code);
-    if (L.eg_code != EG_TRACKING) { tracking_stopped(L); return; }
+    if (L.eg_code != EG_TRACKING) { L.pend = PEND_STOP; return; }  // tracking_stopped!, in lane_close
     L.jtzf0 = L.jtzf1; L.jtzf1 = jump;
     double t = seg_t(L).re;
     if (!(t <= L.eg_start)) return;
@@ -1494,20 +1523,29 @@ __device__ __noinline__ int lane_begin(Lane& L, const hcg_kargs& a, int k) {
         L.q = a.target_params + 2 * HCG_NPAR * g;
     }
 #endif
+    L.pend = PEND_NONE;
     eg_init(L, a.t1);
     L.guard = 0;
     return 1;
 }
 
-__device__ __forceinline__ int lane_ended(const Lane& L) { return L.eg_code != EG_TRACKING; }
+__device__ __forceinline__ int lane_ended(const Lane& L) { return L.eg_code != EG_TRACKING || L.pend != PEND_NONE; }
 
 // One loop iteration of a running path (one tracker step), with the per-path guard.
 __device__ __forceinline__ void lane_iter(Lane& L) {
     eg_step(L);
-    if (++L.guard > 4 * (L.o->max_steps + L.o->max_endgame_steps) + 64) L.eg_code = EG_UNKNOWN;
+    if (++L.guard > 4 * (L.o->max_steps + L.o->max_endgame_steps) + 64) { L.eg_code = EG_UNKNOWN; L.pend = PEND_NONE; }
 }
 
-__device__ __forceinline__ void lane_finish(Lane& L, const hcg_kargs& a, int k, LaneTotals& T) {
+// The end of a path: what is left of its last step and of its endgame, and its record.  The
+// lanes of a wave end their paths in different iterations, but this work (evaluations in
+// double-double, factorizations and a condition estimate, as much as one or two tracker steps) is done
+// when the wave refills, for all lanes that have ended since: otherwise the whole wave would
+// wait through it once per path.  Measured against ending each path at once: parameter batch
+// n = 10, 1,024 paths plain 87.8 -> 82.3 ms, 262,144 paths learned 345.0 -> 332.0 ms.
+__device__ __forceinline__ void lane_close(Lane& L, const hcg_kargs& a, int k, LaneTotals& T) {
+    if (L.pend == PEND_STEP) eg_step(L);
+    if (L.pend == PEND_STOP) { L.pend = PEND_NONE; tracking_stopped(L); }
     write_result(L, a, k);
     T.steps += L.accepted + L.rejected;
     T.newton += L.newton_iters;
