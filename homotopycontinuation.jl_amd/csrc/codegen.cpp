@@ -125,7 +125,7 @@ static std::vector<char> recomputed(const hcg_tape* tp) {
 typedef std::function<std::string(char, int, const std::string&)> StoreFn;
 
 static std::string plain_store(char kind, int idx, const std::string& v) {
-    return std::string(1, kind) + "[" + std::to_string(idx) + "] = " + v + ";";
+    return "pv_st(" + std::string(1, kind) + ", " + std::to_string(idx) + ", " + v + ");";
 }
 
 // Straight-line body of one tape (no signature): inputs x (and pp, pq, pt when pm is
@@ -142,6 +142,7 @@ static void gen_eval(std::ostringstream& os, const hcg_tape* tp, const std::stri
     os << (dd ? "cdd" : "cplx") << "* __restrict__ u";
     if (jac) os << ", cplx* __restrict__ U";
     os << ") {\n";
+    if (pm == PM_DYNAMIC) os << "  hcg_pp ps = hcg_start_params(pp);\n  hcg_gld* qs = (hcg_gld*)pq;\n";
     *flops = gen_eval_body(os, tp, jac, dd, n, pm, fixed, "", plain_store);
     os << "}\n";
 }
@@ -159,12 +160,12 @@ static long gen_eval_body(std::ostringstream& os, const hcg_tape* tp, bool jac, 
     for (int k = 0; k < tp->nparams; k++) {
         std::string v = pfx + "P" + std::to_string(k);
         if (pm == PM_FIXED) lazy_def[tp->params_first + k] = "  const " + std::string(T) + " " + v + " = " + wrap(clit(fixed[2 * k], fixed[2 * k + 1])) + ";\n";
-        else lazy_def[tp->params_first + k] = "  const " + std::string(T) + " " + v + " = " + wrap("par_lerp(pt, pp, pq, " + std::to_string(k) + ")") + ";\n";
+        else lazy_def[tp->params_first + k] = "  const " + std::string(T) + " " + v + " = " + wrap("par_lerp(pt, ps, qs, " + std::to_string(k) + ")") + ";\n";
         nm[tp->params_first + k] = v;
     }
     for (int k = 0; k < tp->nvars; k++) {
         std::string v = pfx + "X" + std::to_string(k);
-        lazy_def[tp->vars_first + k] = "  const " + std::string(T) + " " + v + " = x[" + std::to_string(k) + "];\n";
+        lazy_def[tp->vars_first + k] = "  const " + std::string(T) + " " + v + " = " + (dd ? "x[" + std::to_string(k) + "]" : "pv_ld(x, " + std::to_string(k) + ")") + ";\n";
         nm[tp->vars_first + k] = v;
     }
     auto need = [&](int slot) {
@@ -295,8 +296,8 @@ static long gen_straight_eval_jac(std::ostringstream& os, const hcg_system& G, c
     f += gen_eval_body(os, G.eval_jac, true, false, n, pmG, G.fixed_params, "g",
                        [&](char kind, int idx, const std::string& v) -> std::string {
                            if (!gc[pos(kind, idx)].empty()) return "";
-                           std::string dst = std::string(1, kind) + "[" + std::to_string(idx) + "]";
-                           return dst + " = c_muladd(ts, " + v + ", c_mul(tt, " + dst + "));";
+                           const std::string dst = "pv_ld(" + std::string(1, kind) + ", " + std::to_string(idx) + ")";
+                           return plain_store(kind, idx, "c_muladd(ts, " + v + ", c_mul(tt, " + dst + "))");
                        });
     os << "}\n";
     return f;
@@ -443,7 +444,7 @@ static void gen_dd_interp(std::ostringstream& os, const hcg_tape* tp, const std:
     if (pm == PM_DYNAMIC) os << "const double* __restrict__ pp, const double* __restrict__ pq, cplx pt, ";
     os << "cdd* __restrict__ u) {\n";
     os << "  cdd R[" << std::max(nreg, 1) << "];\n";
-    os << "  DDPar P; P.p = " << (pm == PM_DYNAMIC ? "pp" : "nullptr") << "; P.q = " << (pm == PM_DYNAMIC ? "pq" : "nullptr")
+    os << "  DDPar P; P.p = " << (pm == PM_DYNAMIC ? "(hcg_gld*)pp" : "nullptr") << "; P.q = " << (pm == PM_DYNAMIC ? "(hcg_gld*)pq" : "nullptr")
        << "; P.t = " << (pm == PM_DYNAMIC ? "pt" : "mkc(0.0, 0.0)") << ";\n";
     for (auto& ld : loads) os << "  R[" << ld.first << "] = x[" << (ld.second - tp->nparams) << "];\n";
     os << "  dd_interpret(" << fname << "_code, " << ninstr << ", " << fname << "_const, R, P);\n";
@@ -489,9 +490,10 @@ static void gen_taylor(std::ostringstream& os, const hcg_tape* tp, const std::st
     const bool km1 = pm != PM_DYNAMIC;
     if (km1) os << "cplx* __restrict__ oKm1, ";
     os << "cplx* __restrict__ oK) {\n";
+    if (pm == PM_DYNAMIC) os << "  hcg_pp ps = hcg_start_params(pp);\n  hcg_gld* qs = (hcg_gld*)pq;\n";
     *flops = gen_taylor_body(os, tp, K, n, pm, fixed, "", [km1](int row, const std::string& a, const std::string& b) {
-        std::string r = km1 ? "oKm1[" + std::to_string(row) + "] = " + a + "; " : std::string();
-        return r + "oK[" + std::to_string(row) + "] = " + b + ";";
+        std::string r = km1 ? "pv_st(oKm1, " + std::to_string(row) + ", " + a + "); " : std::string();
+        return r + "pv_st(oK, " + std::to_string(row) + ", " + b + ");";
     });
     os << "}\n";
 }
@@ -515,9 +517,9 @@ static long gen_taylor_body(std::ostringstream& os, const hcg_tape* tp, int K, i
             d = "  const cplx " + nm0 + " = " + clit(fixed[2 * k], fixed[2 * k + 1]) + ";\n";
             s.deg = 0; s.c.push_back(nm0);
         } else {
-            d = "  const cplx " + nm0 + " = par_lerp(pt, pp, pq, " + std::to_string(k) + ");\n";
+            d = "  const cplx " + nm0 + " = par_lerp(pt, ps, qs, " + std::to_string(k) + ");\n";
             std::string nm1 = pfx + "Q" + std::to_string(k);
-            if (K >= 1) d += "  const cplx " + nm1 + " = par_diff(pp, pq, " + std::to_string(k) + ");\n";
+            if (K >= 1) d += "  const cplx " + nm1 + " = par_diff(ps, qs, " + std::to_string(k) + ");\n";
             s.deg = K >= 1 ? 1 : 0; s.c.push_back(nm0);
             if (K >= 1) s.c.push_back(nm1);
         }
@@ -529,7 +531,7 @@ static long gen_taylor_body(std::ostringstream& os, const hcg_tape* tp, int K, i
         std::string& d = lazy_def[tp->vars_first + k];
         for (int j = 0; j < K; j++) {
             std::string nm = pfx + "X" + std::to_string(k) + "_" + std::to_string(j);
-            d += "  const cplx " + nm + " = t" + std::to_string(j) + "[" + std::to_string(k) + "];\n";
+            d += "  const cplx " + nm + " = pv_ld(t" + std::to_string(j) + ", " + std::to_string(k) + ");\n";
             s.c.push_back(nm);
         }
         v[tp->vars_first + k] = s;
@@ -738,16 +740,14 @@ static long gen_straight_taylor(std::ostringstream& os, const hcg_system& G, con
         f += gen_eval_body(os, F.eval, false, false, n, pmF, F.fixed_params, "f",
                            [](char, int i, const std::string& v) { return plain_store('u', i, v); });
         f += gen_eval_body(os, G.eval, false, false, n, pmG, G.fixed_params, "g", [](char, int i, const std::string& v) {
-            std::string d = "u[" + std::to_string(i) + "]";
-            return d + " = c_sub(c_mul(g, " + v + "), " + d + ");";
+            return plain_store('u', i, "c_sub(c_mul(g, " + v + "), pv_ld(u, " + std::to_string(i) + "))");
         });
     } else {
         f += gen_taylor_body(os, F.eval, K, n, pmF, F.fixed_params, "f", [](int i, const std::string& a, const std::string& b) {
-            return "u[" + std::to_string(i) + "] = c_sub(c_mul(omt, " + b + "), " + a + ");";
+            return plain_store('u', i, "c_sub(c_mul(omt, " + b + "), " + a + ")");
         });
         f += gen_taylor_body(os, G.eval, K, n, pmG, G.fixed_params, "g", [](int i, const std::string& a, const std::string& b) {
-            std::string d = "u[" + std::to_string(i) + "]";
-            return d + " = c_add(c_mul(g, c_add(" + a + ", c_mul(t, " + b + "))), " + d + ");";
+            return plain_store('u', i, "c_add(c_mul(g, c_add(" + a + ", c_mul(t, " + b + "))), pv_ld(u, " + std::to_string(i) + "))");
         });
     }
     os << "}\n";
@@ -961,7 +961,7 @@ bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::
     const ParamMode pm = np == 0 ? PM_NONE : (F->fixed_params ? PM_FIXED : PM_DYNAMIC);
     const double* fixed = F->fixed_params;
     std::ostringstream os;
-    os << "// generated by hcgpu codegen (certifier)\n#include \"hcg_arith.h\"\n#include \"hcg_interval.h\"\n";
+    os << "// generated by hcgpu codegen (certifier)\n#define HCG_P_PER_LANE\n#include \"hcg_arith.h\"\n#include \"hcg_interval.h\"\n";
     os << "#define HCG_N " << n << "\n#define HCG_NPAR " << (pm == PM_DYNAMIC ? np : 0) << "\n";
     long f;
     gen_eval(os, F->eval_jac, "certF_eval_jac", true, false, n, pm, fixed, &f);

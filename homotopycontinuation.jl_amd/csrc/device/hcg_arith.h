@@ -407,11 +407,40 @@ HD double ipow(double x, int n) {
 HD double h_of(double a) { return 2 * a * (sqrt(4 * (a * a) + 1) - 2 * a); }
 #define DEPS 2.220446049250313e-16
 
-// Interpreter for double-double tape evaluation (operand >= 0: register, < 0: constant -k-1)
-// Parameters of a parameter homotopy at t: p(t) = t p + (1 - t) q, and the direction
-// p - q of its Taylor series (tp!, src/homotopies/parameter_homotopy.jl:66-87).
-// Both forms are computed and one is selected (no branch): inlined for every parameter of
-// a straight-line body, a branch would split it into hundreds of blocks.
+// Memory of known kind.  Function arguments are generic pointers, and a generic load (flat) may
+// return out of order with every other load in flight, so each wait for one waits for all of
+// them.  A lane's own vectors and matrices live in its private segment and the homotopy's
+// parameters in device memory, so the generated bodies address them as such.  Measured together with
+// the real form of p(t) below, built for one wave per SIMD: parameter batch n = 10, 1,024 paths
+// plain 60.6 -> 48.5 ms, 61,777 plain 177.6 -> 153.7, 262,144 learned 338.0 -> 294.6 (an evaluation
+// with its Jacobian takes 5,092 instructions where it took 7,962).
+typedef __attribute__((address_space(5))) double hcg_pvd;
+typedef const __attribute__((address_space(1))) double hcg_gld;
+HD cplx pv_ld(const cplx* v, int k) {
+    const hcg_pvd* d = (const hcg_pvd*)(const double*)v;
+    return mkc(d[2 * k], d[2 * k + 1]);
+}
+HD void pv_st(cplx* v, int k, cplx z) {
+    hcg_pvd* d = (hcg_pvd*)(double*)v;
+    d[2 * k] = z.re;
+    d[2 * k + 1] = z.im;
+}
+HD double pv_ldd(const double* v, int k) { return ((const hcg_pvd*)v)[k]; }
+HD void pv_std(double* v, int k, double z) { ((hcg_pvd*)v)[k] = z; }
+// The start parameters are one vector for the whole launch: read through the scalar cache (a
+// certifier's parameters are each candidate's own, HCG_P_PER_LANE).
+#ifdef HCG_P_PER_LANE
+typedef hcg_gld* hcg_pp;
+HD hcg_pp hcg_start_params(const double* p) { return (hcg_pp)p; }
+#else
+typedef const __attribute__((address_space(4))) double* hcg_pp;
+HD hcg_pp hcg_start_params(const double* p) {
+    const unsigned long long a = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+    return (hcg_pp)(((unsigned long long)hi << 32) | lo);
+}
+#endif
+
 // A copy of v that the compiler cannot identify with v: the generated code passes the
 // operands of a deliberately repeated computation through it, so that the repetition is not
 // merged back into the first computation (which would keep its result live in between).
@@ -419,22 +448,21 @@ HD cplx hcg_opaque(cplx v) {
     asm volatile("" : "+v"(v.re), "+v"(v.im));
     return v;
 }
-HD cplx par_lerp(cplx t, const double* p, const double* q, int k) {
-    cplx pk = mkc(p[2 * k], p[2 * k + 1]), qk = mkc(q[2 * k], q[2 * k + 1]);
-    cplx rr = c_add(c_scale(t.re, pk), c_scale(1.0 - t.re, qk));
-    cplx rc = c_add(c_mul(t, pk), c_mul(mkc(1.0 - t.re, -t.im), qk));
-    const bool real_t = t.im == 0.0;
-    return mkc(real_t ? rr.re : rc.re, real_t ? rr.im : rc.im);
+// Parameters of a parameter homotopy at t: p(t) = t p + (1 - t) q, and the direction
+// p - q of its Taylor series (tp!, src/homotopies/parameter_homotopy.jl:66-87).  t is real
+// (a path's segment runs between real t1 and t0), so this is the reference's real form.
+template <class P, class Q> HD cplx par_lerp(cplx t, P p, Q q, int k) {
+    return c_add(c_scale(t.re, mkc(p[2 * k], p[2 * k + 1])), c_scale(1.0 - t.re, mkc(q[2 * k], q[2 * k + 1])));
 }
-HD cplx par_diff(const double* p, const double* q, int k) {
+template <class P, class Q> HD cplx par_diff(P p, Q q, int k) {
     return c_sub(mkc(p[2 * k], p[2 * k + 1]), mkc(q[2 * k], q[2 * k + 1]));
 }
 // Operands of the double-double interpreter: >= 0 register, < 0 constant -e-1,
 // >= DD_PBASE homotopy parameter e - DD_PBASE (formed at t when read).
 #define DD_PBASE (1 << 24)
 struct DDPar {
-    const double* p;
-    const double* q;
+    hcg_gld* p;
+    hcg_gld* q;
     cplx t;
 };
 HD cdd dd_fetch(const double* K, const cdd* R, const DDPar& P, int e) {

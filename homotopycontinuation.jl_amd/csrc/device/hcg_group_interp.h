@@ -69,12 +69,9 @@ __device__ __forceinline__ cplx g_gl_c(const double* base, int k) {
     return mkc(d[0], d[1]);
 }
 __device__ __forceinline__ int g_gl_i(const int32_t* base, int k) { return ((const g_glob_i*)base)[k]; }
-// par_lerp (hcg_arith.h) on the values p_k, q_k: the same operations in the same order
+// par_lerp (hcg_arith.h) on the values p_k, q_k: the same operations in the same order (t is real)
 __device__ __forceinline__ cplx g_par_lerp(cplx t, cplx pk, cplx qk) {
-    cplx rr = c_add(c_scale(t.re, pk), c_scale(1.0 - t.re, qk));
-    cplx rc = c_add(c_mul(t, pk), c_mul(mkc(1.0 - t.re, -t.im), qk));
-    const bool real_t = t.im == 0.0;
-    return mkc(real_t ? rr.re : rc.re, real_t ? rr.im : rc.im);
+    return c_add(c_scale(t.re, pk), c_scale(1.0 - t.re, qk));
 }
 
 __device__ __forceinline__ int g_int_imm(int32_t ref) { return ((int)((unsigned)ref << 4)) >> 4; }

@@ -191,14 +191,14 @@ __device__ __noinline__ void lu_factor(Lane& L) {
     const bool sc = L.scaled;
     double r[NN];
     HCG_UNROLL
-    for (int i = 0; i < NN; i++) r[i] = sc ? L.rs[i] : 1.0;
+    for (int i = 0; i < NN; i++) r[i] = sc ? pv_ldd(L.rs, i) : 1.0;
     int piv[NN];
     cplx M[NN][NN];  // M[k][i]: multiplier of row i in column k (i > k)
     HCG_UNROLL
     for (int j = 0; j < NN; j++) {
         cplx c[NN];
         HCG_UNROLL
-        for (int i = 0; i < NN; i++) { cplx a = A[IDX(i, j)]; c[i] = sc ? c_scale(r[i], a) : a; }
+        for (int i = 0; i < NN; i++) { cplx a = pv_ld(A, IDX(i, j)); c[i] = sc ? c_scale(r[i], a) : a; }
         HCG_UNROLL
         for (int k = 0; k < j; k++) reg_swap(c, k, piv[k]);
         HCG_UNROLL
@@ -225,14 +225,14 @@ __device__ __noinline__ void lu_factor(Lane& L) {
             for (int i = j + 1; i < NN; i++) c[i] = c_div(c[i], d);
         }
         HCG_UNROLL
-        for (int i = 0; i <= j; i++) F[IDX(i, j)] = c[i];  // U part: final
+        for (int i = 0; i <= j; i++) pv_st(F, IDX(i, j), c[i]);  // U part: final
         HCG_UNROLL
         for (int i = j + 1; i < NN; i++) M[j][i] = c[i];
     }
     HCG_UNROLL
     for (int k = 0; k < NN; k++) {
         HCG_UNROLL
-        for (int i = k + 1; i < NN; i++) F[IDX(i, k)] = M[k][i];
+        for (int i = k + 1; i < NN; i++) pv_st(F, IDX(i, k), M[k][i]);
     }
     L.factorized = 1;
 }
@@ -243,24 +243,24 @@ __device__ __noinline__ void lu_solve_rs(Lane& L, cplx* x, const cplx* b, const 
     L.flops += FL_SOLVE;
     cplx v[NN];
     HCG_UNROLL
-    for (int i = 0; i < NN; i++) v[i] = rs ? c_scale(rs[i], b[i]) : b[i];
+    for (int i = 0; i < NN; i++) v[i] = rs ? c_scale(pv_ldd(rs, i), pv_ld(b, i)) : pv_ld(b, i);
     HCG_UNROLL
     for (int i = 0; i < NN; i++) reg_swap(v, i, L.ipiv[i]);
     HCG_UNROLL
     for (int j = 0; j < NN; j++) {
         cplx xj = v[j];
         HCG_UNROLL
-        for (int i = j + 1; i < NN; i++) v[i] = c_submul(F[IDX(i, j)], xj, v[i]);
+        for (int i = j + 1; i < NN; i++) v[i] = c_submul(pv_ld(F, IDX(i, j)), xj, v[i]);
     }
     HCG_UNROLL
     for (int j = NN - 1; j >= 0; j--) {
-        cplx xj = c_div(v[j], F[IDX(j, j)]);
+        cplx xj = c_div(v[j], pv_ld(F, IDX(j, j)));
         v[j] = xj;
         HCG_UNROLL
-        for (int i = 0; i < j; i++) v[i] = c_submul(F[IDX(i, j)], xj, v[i]);
+        for (int i = 0; i < j; i++) v[i] = c_submul(pv_ld(F, IDX(i, j)), xj, v[i]);
     }
     HCG_UNROLL
-    for (int i = 0; i < NN; i++) x[i] = v[i];
+    for (int i = 0; i < NN; i++) pv_st(x, i, v[i]);
 }
 #else
 #define HCG_UNROLL
@@ -339,9 +339,9 @@ __device__ __noinline__ void skeel_row_scaling(double* d, const cplx* A, const d
     for (int i = 0; i < NN; i++) r[i] = 0.0;
     HCG_UNROLL
     for (int j = 0; j < NN; j++) {
-        double cj = c[j];
+        double cj = pv_ldd(c, j);
         HCG_UNROLL
-        for (int i = 0; i < NN; i++) r[i] += c_fabs(A[IDX(i, j)]) * cj;
+        for (int i = 0; i < NN; i++) r[i] += c_fabs(pv_ld(A, IDX(i, j))) * cj;
     }
     double m = r[0];
     HCG_UNROLL
@@ -351,13 +351,18 @@ __device__ __noinline__ void skeel_row_scaling(double* d, const cplx* A, const d
     for (int i = 0; i < NN; i++) {
         int e = 0;
         if (isfinite(r[i])) frexp(r[i], &e);
-        d[i] = (double)e < s ? 1.0 : ldexp(1.0, -e);
+        pv_std(d, i, (double)e < s ? 1.0 : ldexp(1.0, -e));
     }
 }
 // weighted / plain inf-norms, src/norm.jl:150-234 (w == nullptr: InfNorm)
 __device__ __noinline__ double norm_inf(const cplx* x, const double* w) {
-    double dmax = w ? c_abs2(c_divr(x[0], w[0])) : c_abs2(x[0]);
-    for (int i = 1; i < NN; i++) dmax = max_fast(dmax, w ? c_abs2(c_divr(x[i], w[i])) : c_abs2(x[i]));
+    double dmax = 0.0;
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) {
+        const cplx z = pv_ld(x, i);
+        const double d = w ? c_abs2(c_divr(z, pv_ldd(w, i))) : c_abs2(z);
+        dmax = i == 0 ? d : max_fast(dmax, d);
+    }
     double d = sqrt(dmax);
     if (isinf(d)) {
         dmax = w ? c_hypot(c_divr(x[0], w[0])) : c_hypot(x[0]);
@@ -367,8 +372,13 @@ __device__ __noinline__ double norm_inf(const cplx* x, const double* w) {
     return d;
 }
 __device__ __noinline__ double dist_inf(const cplx* x, const cplx* y, const double* w) {
-    double dmax = w ? c_abs2(c_divr(c_sub(x[0], y[0]), w[0])) : c_abs2(c_sub(x[0], y[0]));
-    for (int i = 1; i < NN; i++) dmax = max_fast(dmax, w ? c_abs2(c_divr(c_sub(x[i], y[i]), w[i])) : c_abs2(c_sub(x[i], y[i])));
+    double dmax = 0.0;
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) {
+        const cplx z = c_sub(pv_ld(x, i), pv_ld(y, i));
+        const double d = w ? c_abs2(c_divr(z, pv_ldd(w, i))) : c_abs2(z);
+        dmax = i == 0 ? d : max_fast(dmax, d);
+    }
     double d = sqrt(dmax);
     if (isinf(d)) {
         if (w) {

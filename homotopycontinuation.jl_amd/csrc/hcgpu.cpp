@@ -286,8 +286,12 @@ static int hcg_generate_impl(const hcg_homotopy_desc* h, char* buf, size_t bufsz
     return HCG_OK;
 }
 
-// Default register budget of the tracker kernels: waves per SIMD they are built for.
-static const int kDefaultWavesPerEU = 2;
+// Default register budget of the tracker kernels: waves per SIMD they are built for.  A loaded
+// kernel waits for the traffic of its lanes' private state, which a second wave per SIMD doubles
+// and half the registers per lane make larger still.  One against two waves, measured: parameter
+// batch n = 10, 1,024 paths plain 48.5 / 50.5 ms, 61,777 plain 153.7 / 163.7, 262,144 learned 294.6 /
+// 307.8; dense n = 8, 6,561 paths 152.6 / 251.2.
+static const int kDefaultWavesPerEU = 1;
 
 static int build_source(const hcg_homotopy_desc* const* hs, int32_t nsys, int32_t multi, const hcg_build_options* bo,
                         std::string* src, std::vector<hcg::Flops>* fl) {
