@@ -886,10 +886,14 @@ bool generate_multi_source(const hcg_homotopy_desc* const* hs, int nsys, std::st
     const int refill = refill_threshold(m.sys[0].opts);
     int phase = 0, k = -1, s = 0;
     while (true) {
-        int ended = 0;
         const unsigned long long fetch = wave_refill_mask(phase != 1, refill);
-        if (phase != 1) {
-            if (!fetch) continue;
+        int ended = 0;
+        if (phase == 1 || (fetch && phase == 2)) {
+)" << each("if (phase == 1 || @NS::lane_unfinished(@L)) { @NS::lane_iter(@L); ended = @NS::lane_ended(@L); }")
+       << R"(        }
+        if (phase == 1) {
+            if (ended) phase = 2;
+        } else if (fetch) {
             const int kg = wave_fetch(fetch, m.next_path);
             if (phase == 2) {
 )" << each("@NS::lane_close(@L, @A, k, T);")
@@ -899,14 +903,8 @@ bool generate_multi_source(const hcg_homotopy_desc* const* hs, int nsys, std::st
             s = 0;
             while (s + 1 < m.nsys && kg >= m.offset[s + 1]) s++;
             k = kg - m.offset[s];
-            int live = 0;
-)" << each("{ @NS::lane_setup(@L, @A, mw); live = @NS::lane_begin(@L, @A, k); if (live) ended = @NS::lane_ended(@L); }")
-       << R"(            if (!live) continue;
-            phase = 1;
-        } else {
-)" << each("{ @NS::lane_iter(@L); ended = @NS::lane_ended(@L); }")
+)" << each("{ @NS::lane_setup(@L, @A, mw); if (@NS::lane_begin(@L, @A, k)) phase = @NS::lane_ended(@L) ? 2 : 1; }")
        << R"(        }
-        if (ended) phase = 2;
     }
     atomicAdd(&m.sys[0].counters[0], (unsigned long long)T.steps);
     atomicAdd(&m.sys[0].counters[1], (unsigned long long)T.newton);

@@ -30,19 +30,18 @@ extern "C" __global__ void __launch_bounds__(64, HCG_WAVES_PER_EU) hcg_track_ker
     int k = -1;
     while (true) {
         const unsigned long long fetch = wave_refill_mask(phase != 1, refill);
-        if (phase != 1) {
-            if (!fetch) continue;  // wait for more idle lanes of this wave
+        // the rest of an ended path's last step runs beside the other lanes' steps
+        if (phase == 1 || (fetch && phase == 2 && lane_unfinished(L))) lane_iter(L);
+        if (phase == 1) {
+            if (lane_ended(L)) phase = 2;
+        } else if (fetch) {  // else wait for more idle lanes of this wave
             const int kn = wave_fetch(fetch, a.next_path);
             if (phase == 2) lane_close(L, a, k, T);
             phase = 0;
             k = kn;
             if (k >= a.npaths) break;
-            if (!lane_begin(L, a, k)) continue;
-            phase = 1;
-        } else {
-            lane_iter(L);
+            if (lane_begin(L, a, k)) phase = lane_ended(L) ? 2 : 1;
         }
-        if (lane_ended(L)) phase = 2;
     }
     atomicAdd(&a.counters[0], (unsigned long long)T.steps);
     atomicAdd(&a.counters[1], (unsigned long long)T.newton);

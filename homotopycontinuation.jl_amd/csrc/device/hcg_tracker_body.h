@@ -444,6 +444,305 @@ __device__ __noinline__ void jac_ldiv_w(Lane& L, cplx* x, const cplx* b) {
     }
     ws_ldiv(L, x, b);
 }
+// Norm of a vector held in registers: norm_inf(v, w) of the same values (spill: where the
+// overflow fallback finds them).
+#if NN > 1 && NN <= 12
+__device__ __forceinline__ double reg_norm(const cplx (&v)[NN], const double (&w)[NN], cplx* spill, const double* wm) {
+    double dmax = c_abs2(c_divr(v[0], w[0]));
+    HCG_UNROLL
+    for (int i = 1; i < NN; i++) dmax = max_fast(dmax, c_abs2(c_divr(v[i], w[i])));
+    double d = sqrt(dmax);
+    if (isinf(d)) {
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) pv_st(spill, i, v[i]);
+        d = norm_inf(spill, wm);
+    }
+    return d;
+}
+
+// The matrix of one solve as register arrays: M[j][i] is entry (i, j).  With one wave per SIMD
+// (512 registers a lane) the whole matrix stays in registers up to n = 10; otherwise a column is
+// read when it is needed.
+#define HCG_HOLD (HCG_WAVES_PER_EU == 1 && NN <= 10)
+
+// One Newton correction: J Δx = r with J = L.A and r = L.r, L.x̄ -= Δx, returns ‖Δx‖_w.  The same
+// operations on the same values as jac_ldiv_w (`skeel`: row scaling first) or ws_ldiv, norm_inf and the
+// update, in one pass over J: the right-hand side goes through the elimination as one more
+// column, and the factors are stored only when something will use them (`keep`; else they are
+// recomputed from L.A on demand).  upd = 1: no update when the norm is NaN; 2: always.
+// A loaded kernel is bound by the traffic of the lanes' private state (HBM side of L2: 8.5 G lines a
+// launch of the 262,144-path parameter batch with the separate routines, 6.2 G with this one): the
+// pass moves 1.9 KB per lane at n = 10 (3.5 KB with `keep`) where they moved 7.6 KB.  It is inlined
+// down to eg_step, because a called function has to save the 330 registers it needs.
+// Together with the predictor's solves from registers (Factors): 61,777 paths plain 154 -> 131 ms,
+// 262,144 learned 295 -> 247 ms.
+__device__ __forceinline__ double newton_solve(Lane& L, int skeel, int keep, int upd) {
+    L.flops += FL_LU + FL_SOLVE;
+    const cplx* A = L.A;
+    cplx* F = L.LU;
+    double w[NN], rs[NN];
+    cplx M[NN][NN];
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) { w[i] = pv_ldd(L.w, i); rs[i] = 1.0; }
+#if HCG_HOLD
+    HCG_UNROLL
+    for (int j = 0; j < NN; j++) {
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) M[j][i] = pv_ld(A, IDX(i, j));
+    }
+#endif
+    if (skeel) {  // skeel_row_scaling with the weights as column scaling and threshold -30
+        double r[NN];
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) r[i] = 0.0;
+        HCG_UNROLL
+        for (int j = 0; j < NN; j++) {
+            HCG_UNROLL
+            for (int i = 0; i < NN; i++) {
+#if HCG_HOLD
+                const cplx a = M[j][i];
+#else
+                const cplx a = pv_ld(A, IDX(i, j));
+#endif
+                r[i] += c_fabs(a) * w[j];
+            }
+        }
+        double m = r[0];
+        HCG_UNROLL
+        for (int i = 1; i < NN; i++) m = jmax(m, r[i]);
+        const double s = -30.0 + m;
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) {
+            int e = 0;
+            if (isfinite(r[i])) frexp(r[i], &e);
+            rs[i] = (double)e < s ? 1.0 : ldexp(1.0, -e);
+            pv_std(L.rs, i, rs[i]);
+        }
+        L.scaled = 1;
+    }
+#if !HCG_HOLD
+    asm volatile("" ::: "memory");  // the factorization reads A again instead of keeping it in spilled registers
+#endif
+    // lu_factor (left-looking, column by column)
+    int piv[NN];
+    HCG_UNROLL
+    for (int j = 0; j < NN; j++) {
+        cplx c[NN];
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) {
+#if HCG_HOLD
+            c[i] = c_scale(rs[i], M[j][i]);
+#else
+            c[i] = c_scale(rs[i], pv_ld(A, IDX(i, j)));
+#endif
+        }
+        HCG_UNROLL
+        for (int k = 0; k < j; k++) reg_swap(c, k, piv[k]);
+        HCG_UNROLL
+        for (int k = 0; k < j; k++) {
+            cplx ukj = c[k];
+            HCG_UNROLL
+            for (int i = k + 1; i < NN; i++) c[i] = c_submul(M[k][i], ukj, c[i]);
+        }
+        int kp = j;
+        double amax = c_abs2(c[j]);
+        HCG_UNROLL
+        for (int i = j + 1; i < NN; i++) {
+            double absi = c_abs2(c[i]);
+            if (absi > amax) { kp = i; amax = absi; }
+        }
+        piv[j] = kp;
+        reg_swap(c, j, kp);
+        HCG_UNROLL
+        for (int k = 0; k < j; k++) reg_swap(M[k], j, kp);
+        if (amax != 0.0) {
+            cplx d = c[j];
+            HCG_UNROLL
+            for (int i = j + 1; i < NN; i++) c[i] = c_div(c[i], d);
+        }
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) M[j][i] = c[i];
+#if !HCG_HOLD
+        HCG_UNROLL
+        for (int i = 0; i <= j; i++) pv_st(F, IDX(i, j), c[i]);  // U part: final, read back below
+#endif
+    }
+    // lu_solve_rs
+    cplx v[NN];
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) v[i] = c_scale(rs[i], pv_ld(L.r, i));
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) reg_swap(v, i, piv[i]);
+    HCG_UNROLL
+    for (int j = 0; j < NN; j++) {
+        cplx xj = v[j];
+        HCG_UNROLL
+        for (int i = j + 1; i < NN; i++) v[i] = c_submul(M[j][i], xj, v[i]);
+    }
+    if (keep) {
+        HCG_UNROLL
+        for (int j = 0; j < NN; j++) {
+            HCG_UNROLL
+            for (int i = HCG_HOLD ? 0 : j + 1; i < NN; i++) pv_st(F, IDX(i, j), M[j][i]);
+            L.ipiv[j] = piv[j];
+        }
+        L.factorized = 1;
+    }
+    HCG_UNROLL
+    for (int j = NN - 1; j >= 0; j--) {
+#if HCG_HOLD
+#define HCG_U(i, j) M[j][i]
+#else
+#define HCG_U(i, j) pv_ld(F, IDX(i, j))
+#endif
+        cplx xj = c_div(v[j], HCG_U(j, j));
+        v[j] = xj;
+        HCG_UNROLL
+        for (int i = 0; i < j; i++) v[i] = c_submul(HCG_U(i, j), xj, v[i]);
+#undef HCG_U
+    }
+    const double nrm = reg_norm(v, w, L.dx, L.w);
+    if (upd == 2 || !isnan(nrm)) {
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) pv_st(L.xb, i, c_sub(pv_ld(L.xb, i), v[i]));
+    }
+    return nrm;
+}
+
+// The stored factors for solves in a caller: held in registers, read at once, where the matrix
+// fits them (the loads then wait once and not entry by entry), else read as they are used.
+struct Factors {
+#if HCG_HOLD
+    cplx M[NN][NN];
+    __device__ __forceinline__ void load(const cplx* F) {
+        HCG_UNROLL
+        for (int j = 0; j < NN; j++) {
+            HCG_UNROLL
+            for (int i = 0; i < NN; i++) M[j][i] = pv_ld(F, IDX(i, j));
+        }
+    }
+    __device__ __forceinline__ cplx at(int i, int j) const { return M[j][i]; }
+#else
+    const cplx* F;
+    __device__ __forceinline__ void load(const cplx* f) { F = f; }
+    __device__ __forceinline__ cplx at(int i, int j) const { return pv_ld(F, IDX(i, j)); }
+#endif
+    double rs[NN];
+    int piv[NN];
+    __device__ __forceinline__ void load(Lane& L) {
+        load(L.LU);
+        const int sc = L.scaled;
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) {
+            rs[i] = sc ? pv_ldd(L.rs, i) : 1.0;
+            piv[i] = L.ipiv[i];
+        }
+    }
+    __device__ __forceinline__ void solve(cplx (&v)[NN]) const {  // lu_solve_rs
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) v[i] = c_scale(rs[i], v[i]);
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) reg_swap(v, i, piv[i]);
+        HCG_UNROLL
+        for (int j = 0; j < NN; j++) {
+            cplx xj = v[j];
+            HCG_UNROLL
+            for (int i = j + 1; i < NN; i++) v[i] = c_submul(at(i, j), xj, v[i]);
+        }
+        HCG_UNROLL
+        for (int j = NN - 1; j >= 0; j--) {
+            cplx xj = c_div(v[j], at(j, j));
+            v[j] = xj;
+            HCG_UNROLL
+            for (int i = 0; i < j; i++) v[i] = c_submul(at(i, j), xj, v[i]);
+        }
+    }
+};
+
+// ‖J⁻¹ r‖_w with the stored factors (r = L.r).
+__device__ __forceinline__ double solve_norm(Lane& L) {
+    L.flops += FL_SOLVE;
+    Factors f;
+    f.load(L);
+    cplx v[NN];
+    double w[NN];
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) { v[i] = pv_ld(L.r, i); w[i] = pv_ldd(L.w, i); }
+    f.solve(v);
+    return reg_norm(v, w, L.dx, L.w);
+}
+
+// Solves with the stored factors and the negated right-hand side -r (r = L.r), for the
+// predictor: out = x with J x = -r, *norm = ‖x‖_w.  refine: one step of
+// fixed_precision_iterative_refinement!, whose relative correction is returned.
+__device__ __forceinline__ double taylor_solve(Lane& L, cplx* out, double* norm, int refine) {
+    if (!L.factorized) lu_factor(L);
+    L.flops += FL_SOLVE;
+    Factors f;
+    f.load(L);
+    cplx v[NN], x[NN];
+    double w[NN];
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) v[i] = c_neg(pv_ld(L.r, i));
+    double nx = 0.0, ret = 0.0;
+    for (int pass = 0;; pass++) {
+        f.solve(v);
+        HCG_UNROLL
+        for (int i = 0; i < NN; i++) w[i] = pv_ldd(L.w, i);
+        if (pass == 0) {
+            HCG_UNROLL
+            for (int i = 0; i < NN; i++) x[i] = v[i];
+            if (!refine) { nx = reg_norm(x, w, L.tmp, L.w); break; }
+            L.flops += FL_FIXED;
+            HCG_UNROLL
+            for (int i = 0; i < NN; i++) v[i] = mkc(0.0, 0.0);  // A x
+            HCG_UNROLL
+            for (int j = 0; j < NN; j++) {
+                HCG_UNROLL
+                for (int i = 0; i < NN; i++) v[i] = c_muladd(pv_ld(L.A, IDX(i, j)), x[j], v[i]);
+            }
+            HCG_UNROLL
+            for (int i = 0; i < NN; i++) v[i] = c_sub(v[i], c_neg(pv_ld(L.r, i)));
+        } else {
+            HCG_UNROLL
+            for (int i = 0; i < NN; i++) x[i] = c_sub(x[i], v[i]);
+            nx = reg_norm(x, w, L.tmp, L.w);
+            ret = reg_norm(v, w, L.rdx, L.w) / nx;
+            break;
+        }
+    }
+    HCG_UNROLL
+    for (int i = 0; i < NN; i++) pv_st(out, i, x[i]);
+    *norm = nx;
+    return ret;
+}
+#endif
+// The same two operations with the vectors in memory, for the rarer callers and for sizes past
+// the register routines.
+__device__ __noinline__ double newton_solve_mem(Lane& L, int skeel, int upd) {
+    if (skeel) jac_ldiv_w(L, L.dx, L.r);
+    else ws_ldiv(L, L.dx, L.r);
+    const double nrm = norm_inf(L.dx, L.w);
+    if (upd == 2 || !isnan(nrm))
+        for (int k = 0; k < NN; k++) L.xb[k] = c_sub(L.xb[k], L.dx[k]);
+    return nrm;
+}
+__device__ __noinline__ double taylor_solve_mem(Lane& L, cplx* out, double* norm, int refine) {
+    cplx ub[NN];
+    for (int i = 0; i < NN; i++) ub[i] = c_neg(L.r[i]);
+    ws_ldiv(L, out, ub);
+    const double delta = refine ? fixed_refine(L, out, ub, L.w) : 0.0;
+    *norm = norm_inf(out, L.w);
+    return delta;
+}
+#if NN == 1 || NN > 12
+#define newton_solve(L, skeel, keep, upd) newton_solve_mem(L, skeel, upd)
+#define taylor_solve taylor_solve_mem
+__device__ __forceinline__ double solve_norm(Lane& L) {
+    ws_ldiv(L, L.dx, L.r);
+    return norm_inf(L.dx, L.w);
+}
+#endif
 // inverse_inf_norm_est, src/linear_algebra.jl:585-682
 __device__ __noinline__ double inverse_inf_norm_est(Lane& L, const double* dl, const double* dr) {
     if (!L.factorized) lu_factor(L);
@@ -615,8 +914,9 @@ __device__ __forceinline__ NewtRes mkres(int code, double acc, int iters, double
     return R;
 }
 
-// newton!, src/newton_corrector.jl:80-205 (x̄ = L.xb; every iterate aliases it)
-__device__ __noinline__ NewtRes newton(Lane& L, const cplx* x0, cplx t, double mu, double omega, int ext, int accurate_mu, int first_correction) {
+// newton!, src/newton_corrector.jl:80-205 (x̄ = L.xb; every iterate aliases it): the general form, for
+// extended precision and for init_newton!
+__device__ __noinline__ NewtRes newton_any(Lane& L, const cplx* x0, cplx t, double mu, double omega, int ext, int accurate_mu, int first_correction) {
     double a = L.o->a, ha = h_of(a);
     cplx* xb = L.xb;
     if (xb != x0) for (int k = 0; k < NN; k++) xb[k] = x0[k];
@@ -625,31 +925,38 @@ __device__ __noinline__ NewtRes newton(Lane& L, const cplx* x0, cplx t, double m
     for (int i = 0; i <= 10; i++) {
         L.newton_iters++;
         H_eval_jac(L, xb, t, L.r, L.A);
-        if (ext) H_eval_dd(L, xb, t, L.r);
         ws_updated(L);
-        jac_ldiv_w(L, L.dx, L.r);
-        if (ext) iterative_refinement(L, L.dx, L.r, L.w, abar * abar, 3);
-        ndx = norm_inf(L.dx, L.w);
-        if (isnan(ndx)) return mkres(NEWT_SINGULARITY, norm_inf(L.dx, L.w), i + 1, omega, theta, mu_low, ndx0);
-        for (int k = 0; k < NN; k++) xb[k] = c_sub(xb[k], L.dx[k]);
+        if (ext) {
+            H_eval_dd(L, xb, t, L.r);
+            jac_ldiv_w(L, L.dx, L.r);
+            iterative_refinement(L, L.dx, L.r, L.w, abar * abar, 3);
+            ndx = norm_inf(L.dx, L.w);
+            if (!isnan(ndx)) for (int k = 0; k < NN; k++) xb[k] = c_sub(xb[k], L.dx[k]);
+        } else {
+            ndx = newton_solve_mem(L, 1, 1);
+        }
+        if (isnan(ndx)) return mkres(NEWT_SINGULARITY, ndx, i + 1, omega, theta, mu_low, ndx0);
         if (i == 0) ndx0 = ndx;
         if (i == 1) omega = 2 * ndx / (ndx_prev * ndx_prev);
         if (i >= 1) theta = ndx / ndx_prev;
         if ((i >= 1 && theta > abar) || (i == 0 && !first_correction && 0.125 * ndx0 * omega > ha)) {
-            return mkres(NEWT_TERMINATED, norm_inf(L.dx, L.w), i + 1, omega, theta, mu_low, ndx0);
+            return mkres(NEWT_TERMINATED, ndx, i + 1, omega, theta, mu_low, ndx0);
         } else if (omega * (ndx * ndx) < 2 * mu * sqrt(1 - 2 * ha)) {
+            double ndx1;
             H_eval_jac(L, xb, t, L.r, L.A);
             ws_updated(L);
             if (ext) {
                 ws_ldiv(L, L.dx, L.r);
                 mu_low = norm_inf(L.dx, L.w);
                 H_eval_dd(L, xb, t, L.r);
+                ws_ldiv(L, L.dx, L.r);
+                iterative_refinement(L, L.dx, L.r, L.w, abar * abar, 3);
+                for (int k = 0; k < NN; k++) xb[k] = c_sub(xb[k], L.dx[k]);
+                ndx1 = norm_inf(L.dx, L.w);
+            } else {
+                ndx1 = newton_solve_mem(L, 0, 2);
             }
-            ws_ldiv(L, L.dx, L.r);
-            if (ext) iterative_refinement(L, L.dx, L.r, L.w, abar * abar, 3);
-            for (int k = 0; k < NN; k++) xb[k] = c_sub(xb[k], L.dx[k]);
-            double ndx1 = norm_inf(L.dx, L.w);
-            if (isnan(ndx1)) return mkres(NEWT_SINGULARITY, norm_inf(L.dx, L.w), i + 1, omega, theta, mu_low, ndx0);
+            if (isnan(ndx1)) return mkres(NEWT_SINGULARITY, ndx1, i + 1, omega, theta, mu_low, ndx0);
             if (ndx1 > sqrt(ndx)) {
                 theta = ndx1 / ndx;
                 return mkres(NEWT_TERMINATED, ndx1, i + 2, omega, theta, mu_low, ndx0);
@@ -677,6 +984,65 @@ __device__ __noinline__ NewtRes newton(Lane& L, const cplx* x0, cplx t, double m
         if (i >= 1) abar *= abar;
     }
     return mkres(NEWT_MAX_ITERS, mu, 11, omega, theta, mu_low, ndx0);
+}
+
+// newton! in working precision, from L.x̂, as tracker_step calls it.  Each pass of the loop is one
+// evaluation and one solve, for the lanes still iterating and for those in their final
+// simplified step alike, so the wave makes as many passes as its slowest lane and not one more for
+// each iteration at which some lane ends; the accuracy evaluation some lanes need comes
+// after the loop for all of them.
+__device__ __forceinline__ NewtRes newton_step(Lane& L, cplx t, double mu, double omega, int first_correction) {
+    const double a = L.o->a, ha = h_of(a);
+    cplx* xb = L.xb;
+    for (int k = 0; k < NN; k++) xb[k] = L.xh[k];
+    const double mu_low = HCG_NAN;
+    double theta = HCG_NAN, ndx = HCG_NAN, ndx_prev = HCG_NAN, ndx0 = HCG_NAN, ndx1 = HCG_NAN;
+    double abar = a;
+    int i = 0, code = NEWT_MAX_ITERS, iters = 11;
+    bool fin = false;
+    double accuracy = mu;
+    while (true) {
+        L.newton_iters += !fin;
+        H_eval_jac(L, xb, t, L.r, L.A);
+        ws_updated(L);
+        const double d = newton_solve(L, !fin, fin, fin ? 2 : 1);
+        if (!fin) {
+            ndx = d;
+            accuracy = d;
+            iters = i + 1;
+            if (isnan(ndx)) { code = NEWT_SINGULARITY; break; }
+            if (i == 0) ndx0 = ndx;
+            if (i == 1) omega = 2 * ndx / (ndx_prev * ndx_prev);
+            if (i >= 1) theta = ndx / ndx_prev;
+            if ((i >= 1 && theta > abar) || (i == 0 && !first_correction && 0.125 * ndx0 * omega > ha)) {
+                code = NEWT_TERMINATED;
+                break;
+            }
+            if (omega * (ndx * ndx) < 2 * mu * sqrt(1 - 2 * ha)) { fin = true; continue; }
+            ndx_prev = ndx;
+            if (i >= 1) abar *= abar;
+            if (++i > 10) { accuracy = mu; iters = 11; break; }
+        } else {
+            ndx1 = d;
+            accuracy = d;
+            if (isnan(ndx1)) { code = NEWT_SINGULARITY; break; }
+            iters = i + 2;
+            if (ndx1 > sqrt(ndx)) { theta = ndx1 / ndx; code = NEWT_TERMINATED; break; }
+            code = NEWT_CONVERGED;
+            break;
+        }
+    }
+    if (code == NEWT_CONVERGED) {
+        if (ndx1 > 2 * mu) {
+            H_eval(L, xb, t, L.r);
+            accuracy = solve_norm(L);
+        }
+        if (i == 0) {
+            double wb = 2 * ndx / (ndx1 * ndx1);
+            if (wb < omega) omega = wb; else omega *= 0.25;
+        }
+    }
+    return mkres(code, accuracy, iters, omega, theta, mu_low, ndx0);
 }
 
 // init_newton!, src/newton_corrector.jl:207-286
@@ -710,7 +1076,7 @@ __device__ __noinline__ int init_newton(Lane& L, cplx t, int ext, double* omega_
             mu = ndx1;
             double a7 = ipow(a, 7);
             if (omega * mu > a7) {
-                NewtRes rr = newton(L, xb, t, a7 / omega, omega, ext, 1, 0);
+                NewtRes rr = newton_any(L, xb, t, a7 / omega, omega, ext, 1, 0);
                 if (rr.code == NEWT_CONVERGED) { valid = 1; omega = rr.omega; mu = rr.accuracy; }
                 else valid = 0;
             } else {
@@ -753,10 +1119,10 @@ __device__ cplx t_to_s_plane(cplx t, int m) {
 }
 __device__ __forceinline__ cplx cpowi(cplx z, int n) { cplx r = mkc(1.0, 0.0); for (int i = 0; i < n; i++) r = c_mul(r, z); return r; }
 
-// update!(predictor, ...), src/predictor.jl:158-284; xhat may be nullptr
-__device__ __noinline__ void pred_update(Lane& L, cplx t, const cplx* xhat) {
+// update!(predictor, ...), src/predictor.jl:158-284; xhat may be nullptr.  FAST: the register form
+// of the solves, inlined in the caller.
+template <bool FAST> __device__ __forceinline__ void pred_update(Lane& L, cplx t, const cplx* xhat) {
     cplx* u = L.r;
-    cplx xt[NN];
     int m = L.winding;
     for (int i = 0; i < NN; i++) { L.ptx0[i] = L.tx0[i]; L.ptx1[i] = L.tx1[i]; }
     L.pred_prev_t = L.pred_t; L.pred_t = t;
@@ -766,36 +1132,29 @@ __device__ __noinline__ void pred_update(Lane& L, cplx t, const cplx* xhat) {
     for (int i = 0; i < NN; i++) L.tx0[i] = L.x[i];
     L.txn[0] = norm_inf(L.x, L.w);
 
-    H_taylor(L, 1, t, u);
-    for (int i = 0; i < NN; i++) u[i] = c_neg(u[i]);
-    cplx ub[NN];
-    for (int i = 0; i < NN; i++) ub[i] = u[i];
-    ws_ldiv(L, xt, ub);
-    double delta = fixed_refine(L, xt, ub, L.w);
-    L.cond_H_xd = delta / DEPS;
-    if (delta > 1e-10) iterative_refinement(L, xt, ub, nullptr, 1e-10, 5);
-    L.txn[1] = norm_inf(xt, L.w);
-    for (int i = 0; i < NN; i++) L.tx1[i] = xt[i];
-    if (m > 1) {
-        L.hermite = 1;
-        L.order = 4;
-        L.trust_region = L.txn[0] / L.txn[1];
-        if (isnan(L.local_error)) { double q = L.txn[1] / L.txn[0]; L.local_error = q * q * q; }
-        return;
+    // u: H's Taylor coefficient of order K; x^(K) solves J x^(K) = -u
+    double delta = 0.0;
+    for (int K = 1; K <= 3; K++) {
+        cplx* out = K == 1 ? L.tx1 : (K == 2 ? L.tx2 : L.tx3);
+        H_taylor(L, K, t, u);
+        const double d = FAST ? taylor_solve(L, out, &L.txn[K], K == 1) : taylor_solve_mem(L, out, &L.txn[K], K == 1);
+        if (K == 1) {
+            delta = d;
+            L.cond_H_xd = delta / DEPS;
+        }
+        if (delta > (K == 3 ? 1e-4 : 1e-10)) {
+            for (int i = 0; i < NN; i++) u[i] = c_neg(u[i]);
+            iterative_refinement(L, out, u, K == 1 ? nullptr : L.w, K == 3 ? 1e-4 : 1e-10, K == 1 ? 5 : (K == 2 ? 4 : 3));
+            L.txn[K] = norm_inf(out, L.w);
+        }
+        if (m > 1) {
+            L.hermite = 1;
+            L.order = 4;
+            L.trust_region = L.txn[0] / L.txn[1];
+            if (isnan(L.local_error)) { double q = L.txn[1] / L.txn[0]; L.local_error = q * q * q; }
+            return;
+        }
     }
-    H_taylor(L, 2, t, u);
-    for (int i = 0; i < NN; i++) ub[i] = c_neg(u[i]);
-    ws_ldiv(L, xt, ub);
-    if (delta > 1e-10) iterative_refinement(L, xt, ub, L.w, 1e-10, 4);
-    L.txn[2] = norm_inf(xt, L.w);
-    for (int i = 0; i < NN; i++) L.tx2[i] = xt[i];
-
-    H_taylor(L, 3, t, u);
-    for (int i = 0; i < NN; i++) ub[i] = c_neg(u[i]);
-    ws_ldiv(L, xt, ub);
-    if (delta > 1e-4) iterative_refinement(L, xt, ub, L.w, 1e-4, 3);
-    L.txn[3] = norm_inf(xt, L.w);
-    for (int i = 0; i < NN; i++) L.tx3[i] = xt[i];
 
     double tau = HCG_INF;
     for (int i = 0; i < NN; i++) {
@@ -966,7 +1325,7 @@ __device__ __noinline__ int tracker_init(Lane& L, cplx t1, cplx t0) {
     L.pred_t = L.pred_prev_t = mkc(HCG_NAN, 0.0);
     L.pred_s = L.pred_prev_s = mkc(HCG_NAN, 0.0);
     L.trust_region = L.local_error = HCG_NAN;
-    pred_update(L, t, nullptr);
+    pred_update<false>(L, t, nullptr);
     L.tau = L.trust_region;
     double ds = jmax(initial_step_size(L), o->min_step_size);
     seg_propose(L, ds);
@@ -1031,7 +1390,7 @@ __device__ __noinline__ void log_step(Lane& L, const NewtRes& res, int acc) {
 // (outside the singular endgame) returns with L.pend = PEND_STEP after its Newton correction, and
 // the next call does the rest: refinement in double-double and the predictor's update, several
 // ordinary evaluations' work, which lane_close runs for all ended lanes of a wave at once.
-__device__ __noinline__ int tracker_step(Lane& L) {
+__device__ __forceinline__ int tracker_step(Lane& L) {
     const hcg_options* o = L.o;
     NewtRes res;
     double ds0;
@@ -1044,7 +1403,8 @@ __device__ __noinline__ int tracker_step(Lane& L) {
         ds0 = seg_ds(L);
         predict(L, t, dt);
         wnorm_update(L, L.xh);
-        res = newton(L, L.xh, t1, L.mu, L.omega, L.extended_prec, 0, L.accepted == 0);
+        res = L.extended_prec ? newton_any(L, L.xh, t1, L.mu, L.omega, 1, 0, L.accepted == 0)
+                              : newton_step(L, t1, L.mu, L.omega, L.accepted == 0);
         if (res.code == NEWT_CONVERGED && L.last_learned) L.learned_accepted++;
         if (res.code == NEWT_CONVERGED) {
             for (int i = 0; i < NN; i++) L.x[i] = L.xb[i];
@@ -1068,7 +1428,7 @@ __device__ __noinline__ int tracker_step(Lane& L) {
             L.accuracy = refine_current_solution(L, 1e-14, 3);
             L.refined_ext = 1;
         }
-        pred_update(L, seg_t(L), L.xh);
+        pred_update<true>(L, seg_t(L), L.xh);
         L.tau = L.trust_region;
         L.accepted++;
         L.ext_acc += L.extended_prec;
@@ -1417,14 +1777,20 @@ __device__ __noinline__ void eg_step(Lane& L) {
         for (int i = 0; i < NN; i++) L.last_point[i] = L.x[i];
         L.last_t = seg_t(L).re;
     }
+    int jump = 0;
     if (L.singular_endgame) {
         if (L.sing_phase == 0) {
             L.sing_t = seg_t(L).re;
             tracker_init_t0(L, mkc(0.25 * L.sing_t, 0.0));
             L.sing_phase = 1;
         }
+    } else {
+        cplx tp = seg_t1(L);
+        jump = tp.re == 0.0 && tp.im == 0.0;
+    }
+    const int ok = tracker_step(L);
+    if (L.singular_endgame) {
         // one iteration of `while is_tracking(tracker.state.code)`
-        tracker_step(L);
         bool max_steps = false;
         if ((L.steps_eg += 1) >= o->max_endgame_steps) { L.eg_code = EG_MAX_STEPS; max_steps = true; }
         else if (ext_steps(L) - L.ext_steps_eg_start > o->max_endgame_extended_steps) { L.eg_code = EG_MAX_EXT_STEPS; max_steps = true; }
@@ -1433,9 +1799,6 @@ __device__ __noinline__ void eg_step(Lane& L) {
         singular_post(L, max_steps);
         return;
     }
-    cplx tp = seg_t1(L);
-    int jump = tp.re == 0.0 && tp.im == 0.0;
-    int ok = tracker_step(L);
     if (L.pend == PEND_STEP) return;  // the path has reached its end: continued by lane_close
     L.eg_code = tc_to_eg(L.code);
     if (L.eg_code != EG_TRACKING) { L.pend = PEND_STOP; return; }  // tracking_stopped!, in lane_close
@@ -1547,14 +1910,16 @@ __device__ __forceinline__ void lane_iter(Lane& L) {
     if (++L.guard > 4 * (L.o->max_steps + L.o->max_endgame_steps) + 64) { L.eg_code = EG_UNKNOWN; L.pend = PEND_NONE; }
 }
 
-// The end of a path: what is left of its last step and of its endgame, and its record.  The
+// Whether an ended path's last step is to be completed by one more lane_iter before lane_close.
+__device__ __forceinline__ int lane_unfinished(const Lane& L) { return L.pend == PEND_STEP; }
+
+// The end of a path, after its last step: what is left of its endgame, and its record.  The
 // lanes of a wave end their paths in different iterations, but this work (evaluations in
 // double-double, factorizations and a condition estimate, as much as one or two tracker steps) is done
 // when the wave refills, for all lanes that have ended since: otherwise the whole wave would
 // wait through it once per path.  Measured against ending each path at once: parameter batch
 // n = 10, 1,024 paths plain 87.8 -> 82.3 ms, 262,144 paths learned 345.0 -> 332.0 ms.
 __device__ __forceinline__ void lane_close(Lane& L, const hcg_kargs& a, int k, LaneTotals& T) {
-    if (L.pend == PEND_STEP) eg_step(L);
     if (L.pend == PEND_STOP) { L.pend = PEND_NONE; tracking_stopped(L); }
     write_result(L, a, k);
     T.steps += L.accepted + L.rejected;
@@ -1570,3 +1935,6 @@ __device__ __forceinline__ void lane_close(Lane& L, const hcg_kargs& a, int k, L
 #undef FL_MIXED
 #undef FL_FIXED
 #undef HCG_UNROLL
+#undef HCG_HOLD
+#undef newton_solve
+#undef taylor_solve

@@ -54,7 +54,7 @@ typedef struct hcg_options {
     double learned_inf_logit;
     int32_t refill_idle;         /* scheduling (no counterpart in the reference): finished lanes of a
                                     wave start their next paths together once at least this many of
-                                    the wave's lanes are idle, or all are; 0 = default 8, 1 = at once */
+                                    the wave's lanes are idle, or all are; 0 = default 12, 1 = at once */
     int32_t reserved_i;
 } hcg_options;
 
