@@ -20,6 +20,7 @@ struct MlpWork {
     float* w = nullptr;        // cap * 2
     float* pred = nullptr;     // cap * 2
     float* loss = nullptr;     // 1
+    float* part = nullptr;     // partial gradients, a row per workgroup
     int32_t* perm = nullptr;   // cap
     long cap = 0;
 };
