@@ -885,7 +885,7 @@ bool generate_multi_source(const hcg_homotopy_desc* const* hs, int nsys, std::st
     LaneTotals T = {0, 0, 0, 0.0};
     const int refill = refill_threshold(m.sys[0].opts);
     int phase = 0, k = -1, s = 0;
-    while (true) {
+    while ((int)threadIdx.x < m.sys[0].lanes) {
         const unsigned long long fetch = wave_refill_mask(phase != 1, refill);
         int ended = 0;
         if (phase == 1 || (fetch && phase == 2)) {
@@ -906,10 +906,10 @@ bool generate_multi_source(const hcg_homotopy_desc* const* hs, int nsys, std::st
 )" << each("{ @NS::lane_setup(@L, @A, mw); if (@NS::lane_begin(@L, @A, k)) phase = @NS::lane_ended(@L) ? 2 : 1; }")
        << R"(        }
     }
-    atomicAdd(&m.sys[0].counters[0], (unsigned long long)T.steps);
-    atomicAdd(&m.sys[0].counters[1], (unsigned long long)T.newton);
-    atomicAdd(&m.sys[0].counters[2], (unsigned long long)T.flops);
-    atomicAdd(&m.sys[0].counters[3], (unsigned long long)T.lacc);
+    wave_add(&m.sys[0].counters[0], (unsigned long long)T.steps);
+    wave_add(&m.sys[0].counters[1], (unsigned long long)T.newton);
+    wave_add(&m.sys[0].counters[2], (unsigned long long)T.flops);
+    wave_add(&m.sys[0].counters[3], (unsigned long long)T.lacc);
 }
 )";
     *src = os.str();

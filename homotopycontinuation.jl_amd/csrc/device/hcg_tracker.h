@@ -28,7 +28,7 @@ extern "C" __global__ void __launch_bounds__(64, HCG_WAVES_PER_EU) hcg_track_ker
     const int refill = refill_threshold(a.opts);
     int phase = 0;  // 0: idle, 1: tracking, 2: path k has ended and is not closed yet
     int k = -1;
-    while (true) {
+    while ((int)threadIdx.x < a.lanes) {
         const unsigned long long fetch = wave_refill_mask(phase != 1, refill);
         // the rest of an ended path's last step runs beside the other lanes' steps
         if (phase == 1 || (fetch && phase == 2 && lane_unfinished(L))) lane_iter(L);
@@ -43,8 +43,8 @@ extern "C" __global__ void __launch_bounds__(64, HCG_WAVES_PER_EU) hcg_track_ker
             if (lane_begin(L, a, k)) phase = lane_ended(L) ? 2 : 1;
         }
     }
-    atomicAdd(&a.counters[0], (unsigned long long)T.steps);
-    atomicAdd(&a.counters[1], (unsigned long long)T.newton);
-    atomicAdd(&a.counters[2], (unsigned long long)T.flops);
-    atomicAdd(&a.counters[3], (unsigned long long)T.lacc);
+    wave_add(&a.counters[0], (unsigned long long)T.steps);
+    wave_add(&a.counters[1], (unsigned long long)T.newton);
+    wave_add(&a.counters[2], (unsigned long long)T.flops);
+    wave_add(&a.counters[3], (unsigned long long)T.lacc);
 }
