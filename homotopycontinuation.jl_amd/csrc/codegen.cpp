@@ -949,6 +949,142 @@ static void gen_cert_interp(std::ostringstream& os, const hcg_tape* tp, const st
     os << "}\n";
 }
 
+// A tape split at the values that depend on its parameters only: `main` takes each such value that the
+// rest of the tape (or an output) reads as a parameter of its own, and cones[c] is the program of one of
+// them, over the original parameters.  The operations of every value are the tape's own, so evaluating
+// the cones once per parameter vector and `main` per point gives the unsplit tape's results.
+struct SplitTape {
+    std::vector<int32_t> instr, u_assign, U_assign;
+    hcg_tape main;
+    std::vector<InterpPlan> cones;
+    int nreg = 0;  // registers of the largest cone
+};
+// Below this many parameter-only operations the tape stays whole.
+static const int kSplitMin = 32;
+
+static bool split_tape(const hcg_tape* tp, const std::vector<std::pair<int, int>>& outs, SplitTape* S) {
+    const int np = tp->nparams;
+    std::vector<int> def_of(tp->tape_space + 1, -1);  // slot -> definition: parameters, variables, instructions
+    int nd = 0;
+    for (int k = 0; k < np; k++) def_of[tp->params_first + k] = nd++;
+    for (int k = 0; k < tp->nvars; k++) def_of[tp->vars_first + k] = nd++;
+    const int first = nd;
+    int ninstr = 0;
+    while (ninstr < tp->ninstr && tp->instr[6 * ninstr + 4] != OP_STOP) ninstr++;
+    // per definition: the instruction's input definitions (-1: constant or none); parameter-only flag
+    std::vector<std::array<int, 4>> in(ninstr);
+    std::vector<char> ponly(first + ninstr, 0);
+    for (int k = 0; k < np; k++) ponly[k] = 1;
+    int npo = 0;
+    for (int i = 0; i < ninstr; i++) {
+        const int32_t* I = tp->instr + 6 * i;
+        bool po = true;
+        for (int q = 0; q < 4; q++) {
+            in[i][q] = -1;
+            if (q >= arity(I[4]) || (I[4] == OP_POW_INT && q == 1) || I[q] <= tp->nconst) continue;
+            in[i][q] = def_of[I[q]];
+            po = po && ponly[in[i][q]];
+        }
+        ponly[first + i] = po;
+        npo += po;
+        def_of[I[5]] = first + i;
+    }
+    if (npo < kSplitMin) return false;
+    std::vector<int> coef(first + ninstr, -1), order;
+    auto need = [&](int d) { if (d >= 0 && ponly[d] && coef[d] < 0) { coef[d] = (int)order.size(); order.push_back(d); } };
+    for (int i = 0; i < ninstr; i++)
+        if (!ponly[first + i]) for (int q = 0; q < 4; q++) need(in[i][q]);
+    for (auto& o : outs) if (o.second > tp->nconst) need(def_of[o.second]);
+    // the main tape: constants, coefficients, variables, then one slot per instruction
+    const int nc = (int)order.size(), vf = tp->nconst + nc + 1;
+    std::vector<int> slot(first + ninstr, 0);
+    for (int d = 0; d < first + ninstr; d++) if (coef[d] >= 0) slot[d] = tp->nconst + 1 + coef[d];
+    for (int k = 0; k < tp->nvars; k++) slot[np + k] = vf + k;
+    int next = vf + tp->nvars;
+    for (int i = 0; i < ninstr; i++) {
+        if (ponly[first + i]) continue;
+        const int32_t* I = tp->instr + 6 * i;
+        slot[first + i] = next++;
+        for (int q = 0; q < 4; q++) S->instr.push_back(in[i][q] >= 0 ? slot[in[i][q]] : I[q]);
+        S->instr.push_back(I[4]);
+        S->instr.push_back(slot[first + i]);
+    }
+    S->main = *tp;
+    S->main.instr = S->instr.data();
+    S->main.ninstr = (int32_t)(S->instr.size() / 6);
+    S->main.params_first = tp->nconst + 1;
+    S->main.nparams = nc;
+    S->main.vars_first = vf;
+    S->main.tape_space = next;
+    for (int i = 0; i < tp->nu; i++) {
+        const int s = tp->u_assign[2 * i + 1];
+        S->u_assign.push_back(tp->u_assign[2 * i]);
+        S->u_assign.push_back(s <= tp->nconst ? s : slot[def_of[s]]);
+    }
+    for (int i = 0; i < tp->nU; i++) {
+        const int s = tp->U_assign[2 * i + 1];
+        S->U_assign.push_back(tp->U_assign[2 * i]);
+        S->U_assign.push_back(s <= tp->nconst ? s : slot[def_of[s]]);
+    }
+    S->main.u_assign = S->u_assign.data();
+    S->main.U_assign = S->U_assign.data();
+    // the cones, each with the instructions it reaches; shared ones are repeated
+    long total = 0;
+    for (int d : order) {
+        std::vector<char> use(first + ninstr, 0);
+        use[d] = 1;
+        for (int i = ninstr - 1; i >= 0; i--)
+            if (use[first + i]) for (int q = 0; q < 4; q++) if (in[i][q] >= 0) use[in[i][q]] = 1;
+        std::vector<int32_t> ci;
+        for (int i = 0; i < ninstr; i++) {
+            if (!use[first + i]) continue;
+            const int32_t* I = tp->instr + 6 * i;
+            // one slot per definition, past the inputs
+            for (int q = 0; q < 4; q++) ci.push_back(in[i][q] < 0 ? I[q] : in[i][q] < np ? tp->params_first + in[i][q] : tp->tape_space + 1 + in[i][q] - first);
+            ci.push_back(I[4]);
+            ci.push_back(tp->tape_space + 1 + i);
+        }
+        hcg_tape c = *tp;
+        c.instr = ci.data();
+        c.ninstr = (int32_t)(ci.size() / 6);
+        c.tape_space = tp->tape_space + 1 + ninstr;
+        const int os = d < np ? tp->params_first + d : tp->tape_space + 1 + d - first;
+        S->cones.push_back(plan_interp(&c, {{0, os}}, 1, PM_DYNAMIC, nullptr, 1 << 24));
+        S->nreg = std::max(S->nreg, S->cones.back().nreg);
+        total += c.ninstr;
+        if (total > 4L * ninstr + 64) return false;  // heavily shared: the cones would repeat too much
+    }
+    return true;
+}
+
+// The cones' tables and the device function <fname>_coef(T, c, PD, IP, BP, D, I, B): coefficient c of one parameter
+// vector in double-double (from the point), intervals and balls.
+static void emit_cones(std::ostringstream& os, const hcg_tape* tp, const std::string& fname, const SplitTape& S, bool dd) {
+    InterpPlan all;
+    for (int k = 0; k < 2 * tp->nconst; k++) all.consts.push_back(tp->constants[k]);
+    std::ostringstream off, outp;
+    for (auto& c : S.cones) {
+        off << all.code.size() / 6 << ",";
+        outp << c.out_operand[0] << ",";
+        all.code.insert(all.code.end(), c.code.begin(), c.code.end());
+    }
+    emit_tables(os, fname + "_cone", all);
+    os << "__constant__ int " << fname << "_off[] = {" << off.str() << all.code.size() / 6 << "};\n";
+    os << "__constant__ int " << fname << "_out[] = {" << outp.str() << "0};\n";
+    const std::string args = fname + "_cone_code + 6 * " + fname + "_off[c], " + fname + "_off[c + 1] - " + fname + "_off[c], " + fname + "_cone_const";
+    const std::string nr = std::to_string(std::max(S.nreg, 1));
+    os << "__device__ __noinline__ void " << fname << "_coef(int c, const double* P, const double* IP, const double* BP, double* D, double* I, double* B) {\n";
+    if (dd) {
+        os << "  { cdd R[" << nr << "]; DDPar Q; Q.p = (hcg_gld*)P; Q.q = (hcg_gld*)P; Q.t = mkc(0.0, 0.0);\n    dd_interpret(" << args << ", R, Q);\n"
+           << "    const cdd v = dd_fetch(" << fname << "_cone_const, R, Q, " << fname << "_out[c]);\n"
+           << "    double* o = D + 4 * c; o[0] = v.re.hi; o[1] = v.re.lo; o[2] = v.im.hi; o[3] = v.im.lo; }\n";
+    }
+    os << "  { icplx R[" << nr << "];\n    ci_interpret(" << args << ", R, IP);\n    const icplx v = ci_fetch(" << fname << "_cone_const, R, IP, " << fname << "_out[c]);\n"
+       << "    double* o = I + 4 * c; o[0] = v.re.lo; o[1] = v.re.hi; o[2] = v.im.lo; o[3] = v.im.hi; }\n"
+       << "  { cball R[" << nr << "];\n    cb_interpret(" << args << ", R, BP);\n    const cball v = cb_fetch(" << fname << "_cone_const, R, BP, " << fname << "_out[c]);\n"
+       << "    cb_st(B, c, v); }\n}\n";
+}
+
 bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::string* err) {
     if (!F || !F->eval || !F->eval_jac) { *err = "NULL system"; return false; }
     if (n < 1 || n > HCG_MAX_N) { *err = "system size out of range (1.." + std::to_string(HCG_MAX_N) + ")"; return false; }
@@ -963,14 +1099,30 @@ bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::
     os << "#define HCG_N " << n << "\n#define HCG_NPAR " << (pm == PM_DYNAMIC ? np : 0) << "\n";
     long f;
     gen_eval(os, F->eval_jac, "certF_eval_jac", true, false, n, pm, fixed, &f);
-    gen_dd_interp(os, F->eval, "certF_eval_dd", n, pm, fixed, &f);
-    gen_cert_interp(os, F->eval, "cert_ieval", false, n, pm, fixed, false);
-    gen_cert_interp(os, F->eval_jac, "cert_ijac", true, n, pm, fixed, false);
-    gen_cert_interp(os, F->eval, "cert_beval", false, n, pm, fixed, true);
-    gen_cert_interp(os, F->eval_jac, "cert_bjac", true, n, pm, fixed, true);
+    // coefficients that depend on the parameters only are evaluated once per parameter vector
+    // (hcg_cert_coef_kernel) when both tapes split; they are most of a system whose coefficients are
+    // formed from its parameters (3,400 of 3,900 operations in the n = 10 parameter system)
+    SplitTape se, sj;
+    std::vector<std::pair<int, int>> oe, oj;
+    for (int i = 0; i < F->eval->nu; i++) oe.push_back({F->eval->u_assign[2 * i] - 1, F->eval->u_assign[2 * i + 1]});
+    for (int i = 0; i < F->eval_jac->nU; i++) oj.push_back({F->eval_jac->U_assign[2 * i] - 1, F->eval_jac->U_assign[2 * i + 1]});
+    const bool split = pm == PM_DYNAMIC && split_tape(F->eval, oe, &se) && split_tape(F->eval_jac, oj, &sj);
+    const hcg_tape* te = split ? &se.main : F->eval;
+    const hcg_tape* tj = split ? &sj.main : F->eval_jac;
+    os << "#define HCG_CERT_NCE " << (split ? se.main.nparams : 0) << "\n#define HCG_CERT_NCJ " << (split ? sj.main.nparams : 0) << "\n";
+    gen_dd_interp(os, te, "certF_eval_dd", n, pm, fixed, &f);
+    gen_cert_interp(os, te, "cert_ieval", false, n, pm, fixed, false);
+    gen_cert_interp(os, tj, "cert_ijac", true, n, pm, fixed, false);
+    gen_cert_interp(os, te, "cert_beval", false, n, pm, fixed, true);
+    gen_cert_interp(os, tj, "cert_bjac", true, n, pm, fixed, true);
+    if (split) {
+        emit_cones(os, F->eval, "certE", se, true);
+        emit_cones(os, F->eval_jac, "certJ", sj, false);
+    }
     const std::string pa = pm == PM_DYNAMIC ? "P, P, mkc(0.0, 0.0), " : "";
     os << "HD void cert_eval_jac(const cplx* x, const double* P, cplx* u, cplx* U) { certF_eval_jac(x, " << pa << "u, U); }\n";
-    os << "HD void cert_eval_dd(const cdd* x, const double* P, cdd* u) { certF_eval_dd(x, " << pa << "u); }\n";
+    os << "HD void cert_eval_dd(const cdd* x, const double* P, cdd* u) { certF_eval_dd(x, "
+       << (split ? "P, nullptr, mkc(0.0, 0.0), " : pa) << "u); }\n";
     os << "#include \"hcg_certify.h\"\n";
     *src = os.str();
     return true;

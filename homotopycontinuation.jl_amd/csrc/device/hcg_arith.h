@@ -466,6 +466,12 @@ struct DDPar {
     cplx t;
 };
 HD cdd dd_fetch(const double* K, const cdd* R, const DDPar& P, int e) {
+#ifdef HCG_P_PER_LANE
+    if (e >= DD_PBASE && !P.q) {  // a certifier's coefficient tables hold double-double values
+        hcg_gld* c = P.p + 4 * (e - DD_PBASE);
+        return mkcdd(mkdd(c[0], c[1]), mkdd(c[2], c[3]));
+    }
+#endif
     if (e >= DD_PBASE) return cdd_from(par_lerp(P.t, P.p, P.q, e - DD_PBASE));
     return e >= 0 ? R[e] : cdd_from(mkc(K[2 * (-e - 1)], K[2 * (-e - 1) + 1]));
 }

@@ -21,7 +21,11 @@
 //   cert_ieval(X, IP, u)        F on a box,  cert_ijac(X, IP, U)  ∂F/∂x on a box
 //   cert_beval(x, BP, u)        F at a double-double point in double-double balls
 //   cert_bjac(x, BP, U)         ∂F/∂x at that point, the same way
-// with P the parameter point (HCG_NPAR complex), IP its box (HCG_NPAR × 4 doubles) and BP
+// and, where the tapes are split (HCG_CERT_NCE > 0), certE_coef / certJ_coef, the coefficients that depend on
+// the parameters only: cert_eval_dd and the interval and ball functions then take tables of
+// those coefficients in place of the parameters, filled once per parameter vector by
+// hcg_cert_coef_kernel.
+// P is the parameter point (HCG_NPAR complex), IP its box (HCG_NPAR × 4 doubles) and BP
 // its double-double ball (HCG_NPAR × 6 doubles).
 #pragma once
 #include "hcg_cert_kargs.h"
@@ -217,9 +221,36 @@ __device__ __noinline__ void cert_refine_dd(cdd* xd, const cplx* C, const double
     }
 }
 
+#if HCG_CERT_NCE > 0
+// A candidate's time is the latency of its interpreted evaluations (registers in private memory), so what
+// does not depend on the candidate is taken out of them: 16,000 candidates of the n = 10 parameter
+// system on 16 parameter vectors 47.2 -> 8.0 ms for the whole call.
+// Coefficient tables of one parameter vector, in doubles from its start: double-double values, boxes and
+// balls of the evaluation's coefficients, then boxes and balls of the Jacobian's.
+#define CERT_IE (4 * HCG_CERT_NCE)
+#define CERT_BE (8 * HCG_CERT_NCE)
+#define CERT_IJ (14 * HCG_CERT_NCE)
+#define CERT_BJ (14 * HCG_CERT_NCE + 4 * HCG_CERT_NCJ)
+#define CERT_COEF (14 * HCG_CERT_NCE + 10 * HCG_CERT_NCJ)
+// One lane per coefficient and parameter vector.
+extern "C" __global__ void __launch_bounds__(64) hcg_cert_coef_kernel(hcg_cert_kargs a) {
+    const int per = HCG_CERT_NCE + HCG_CERT_NCJ;
+    const long t = (long)blockIdx.x * 64 + threadIdx.x;
+    if (t >= (long)(a.g1 - a.g0) * per) return;
+    const long s = t / per, g = a.g0 + s;
+    const int c = (int)(t % per);
+    const double* P = a.params + 2 * HCG_NPAR * g;
+    const double* IP = a.params_ival + 4 * HCG_NPAR * g;
+    const double* BP = a.params_ball + 6 * HCG_NPAR * g;
+    double* T = a.coef + CERT_COEF * s;
+    if (c < HCG_CERT_NCE) certE_coef(c, P, IP, BP, T, T + CERT_IE, T + CERT_BE);
+    else certJ_coef(c - HCG_CERT_NCE, P, IP, BP, T, T + CERT_IJ, T + CERT_BJ);
+}
+#endif
+
 // Four waves per SIMD (128 registers per lane): the kernel is latency-bound on its private
-// memory, and occupancy beats registers here.  Measured on 262,144 candidates at n = 10: 176 ms
-// at one wave per SIMD, 109 ms at two, 81 ms at four, 127 ms at eight.
+// memory, and occupancy beats registers here.  Measured on 262,144 candidates at n = 10 with whole tapes:
+// 176 ms at one wave per SIMD, 109 ms at two, 81 ms at four, 127 ms at eight.
 extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_kargs a) {
     const long k = (long)blockIdx.x * 64 + threadIdx.x;
     if (k >= a.nsol) return;
@@ -227,6 +258,14 @@ extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_
     const double* P = a.params ? a.params + 2 * HCG_NPAR * g : nullptr;
     const double* IP = a.params_ival ? a.params_ival + 4 * HCG_NPAR * g : nullptr;
     const double* BP = a.params_ball ? a.params_ball + 6 * HCG_NPAR * g : nullptr;
+    // what the double-double, interval and ball evaluations read: the parameters, or coefficient tables
+#if HCG_CERT_NCE > 0
+    if (g < a.g0 || g >= a.g1) return;
+    const double* T = a.coef + (long)CERT_COEF * (g - a.g0);
+    const double *PD = T, *IE = T + CERT_IE, *IJ = T + CERT_IJ, *BE = T + CERT_BE, *BJ = T + CERT_BJ;
+#else
+    const double *PD = P, *IE = IP, *IJ = IP, *BE = BP, *BJ = BP;
+#endif
     cplx x[CN], r[CN], LU[CN * CN];
     int ipiv[CN];
     for (int i = 0; i < CN; i++) x[i] = mkc(a.candidates[2 * (k * CN + i)], a.candidates[2 * (k * CN + i) + 1]);
@@ -242,7 +281,7 @@ extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_
             cert_eval_jac(x, P, r, LU);
             cdd xe[CN], re[CN];
             for (int i = 0; i < CN; i++) xe[i] = cdd_from(x[i]);
-            cert_eval_dd(xe, P, re);
+            cert_eval_dd(xe, PD, re);
             for (int i = 0; i < CN; i++) r[i] = cdd_round(re[i]);
             cert_lu(LU, ipiv);
             cert_lu_solve(LU, ipiv, r);
@@ -281,23 +320,23 @@ extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_
         X[i] = ic_pt(x[i]);
         xd[i] = cdd_from(x[i]);
     }
-    cert_ieval(X, IP, R0);  // r₀ = F([x̃]) in FP64 intervals
+    cert_ieval(X, IE, R0);  // r₀ = F([x̃]) in FP64 intervals
     double* b1 = a.box1 + 4 * k * CN;
     double* b0 = a.box0 + 4 * k * CN;
-    KrawczykOut o = cert_krawczyk(xd, C, R0, IP, false, b1, b0);
+    KrawczykOut o = cert_krawczyk(xd, C, R0, IJ, false, b1, b0);
     int prec = 53;
     if (!o.certified && a.extended) {
         // Extended precision (the role of the reference's Arb retry, extended_prec_certify_solution
         // and arb_ε_inflation_krawczyk, src/certification.jl:1116-1218, 1289-1394): x̃ becomes a
         // double-double point refined with double-double ball residuals and the test runs again;
         // if it still fails, C is recomputed from a double-double Jacobian and it runs once more.
-        cert_refine_dd(xd, C, BP, R0);
-        o = cert_krawczyk(xd, C, R0, IP, true, b1, b0);
+        cert_refine_dd(xd, C, BE, R0);
+        o = cert_krawczyk(xd, C, R0, IJ, true, b1, b0);
         prec = 106;
         if (!o.certified) {
-            cert_dd_inverse(xd, BP, C);
-            cert_refine_dd(xd, C, BP, R0);
-            o = cert_krawczyk(xd, C, R0, IP, true, b1, b0);
+            cert_dd_inverse(xd, BJ, C);
+            cert_refine_dd(xd, C, BE, R0);
+            o = cert_krawczyk(xd, C, R0, IJ, true, b1, b0);
         }
     }
     for (int i = 0; i < CN; i++) {

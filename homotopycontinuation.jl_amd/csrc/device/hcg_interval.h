@@ -233,6 +233,11 @@ HD cball cb_ddpt(cdd z) { return mkcb(mkdb(z.re, 0.0), mkdb(z.im, 0.0)); }
 HD cball cb_ld(const double* B, int k) {  // parameter k of a packed (re hi, re lo, re rad, im hi, im lo, im rad) array
     return mkcb(mkdb(mkdd(B[6 * k], B[6 * k + 1]), B[6 * k + 2]), mkdb(mkdd(B[6 * k + 3], B[6 * k + 4]), B[6 * k + 5]));
 }
+HD void cb_st(double* B, int k, cball z) {
+    double* o = B + 6 * k;
+    o[0] = z.re.m.hi; o[1] = z.re.m.lo; o[2] = z.re.r;
+    o[3] = z.im.m.hi; o[4] = z.im.m.lo; o[5] = z.im.r;
+}
 HD cball cb_nan() { return mkcb(mkdb(mkdd(HCG_NAN, 0.0), HCG_INF), mkdb(mkdd(HCG_NAN, 0.0), HCG_INF)); }
 HD icplx cb_to_ic(cball z) { return mkic(db_to_ival(z.re), db_to_ival(z.im)); }
 HD cball cb_neg(cball a) { return mkcb(db_neg(a.re), db_neg(a.im)); }
