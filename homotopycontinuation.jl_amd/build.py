@@ -62,7 +62,7 @@ def hipcc():
 
 
 SOURCES = ["hcgpu.cpp", "codegen.cpp", "mlp.hip", "noalloc.hip", "group_sched.cpp", "group.cpp", "group_kernel.hip",
-           "group_kernel32.hip"]
+           "group_kernel32.hip", "group_kernel32_wide.hip"]
 # -ffp-contract=off: FMAs only where the code writes fma(), the arithmetic contract the oracle and
 # the hipRTC-compiled kernels share (results equal the oracle's bit for bit)
 FLAGS = ["-O3", "-fPIC", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-Xclang", "-target-feature",

@@ -213,7 +213,8 @@ __device__ __forceinline__ void hcg_group_run(const hcg_multi_kargs& m, const hc
     long long steps = 0, newton = 0, lacc = 0;
     int k = -1, s = 0;
     long evals = 0;
-    while (true) {
+    // a small batch uses the first groups of each wave only (the launcher's choice)
+    while ((int)(__lane_id() / GL) < m.sys[0].lanes) {
         if (k < 0) {
             int kk = 0;
             if (T.r == 0) kk = atomicAdd(m.next_path, 1);

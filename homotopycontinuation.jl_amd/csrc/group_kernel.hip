@@ -31,9 +31,9 @@ template <int NN> hipError_t allow_lds(size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-hipError_t group_launch(int nn, int grid, int lds_per_path, bool mlp_lds, hipStream_t stream,
+hipError_t group_launch(int nn, int grid, bool one_per_cu, int lds_per_path, bool mlp_lds, hipStream_t stream,
                         const hcg_multi_kargs& m, const hcg_gsys* d_sys) {
-    if (nn > 16) return group_launch32(nn, grid, lds_per_path, mlp_lds, stream, m, d_sys);
+    if (nn > 16) return group_launch32(nn, grid, one_per_cu, lds_per_path, mlp_lds, stream, m, d_sys);
     // LDS: the step network's BF16 weights (learned step only), then each group's registers
     const size_t shmem = (mlp_lds ? (size_t)kMlpLdsBytes : 0) + (size_t)(kBlock / HCG_GROUP_LANES) * lds_per_path;
     hipError_t e = nn == 4 ? allow_lds<4>(shmem) : nn == 8 ? allow_lds<8>(shmem) : nn == 12 ? allow_lds<12>(shmem)

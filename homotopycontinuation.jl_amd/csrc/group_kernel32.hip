@@ -31,10 +31,11 @@ template <int NN> hipError_t allow_lds32(size_t bytes) {
 
 namespace hcg {
 
-hipError_t group_launch32(int nn, int grid, int lds_per_path, bool mlp_lds, hipStream_t stream,
+hipError_t group_launch32(int nn, int grid, bool one_per_cu, int lds_per_path, bool mlp_lds, hipStream_t stream,
                           const hcg_multi_kargs& m, const hcg_gsys* d_sys) {
     const size_t shmem = (mlp_lds ? (size_t)HCG_GROUP_MLP_LDS : 0) + (size_t)(kBlock / GL) * lds_per_path;
     if (nn != 24) return hipErrorInvalidValue;
+    if (one_per_cu) return group_launch32_wide(grid, shmem, lds_per_path, stream, m, d_sys);
     hipError_t e = allow_lds32<24>(shmem);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(hcg_group_kernel32<24>, dim3(grid), dim3(kBlock), shmem, stream, m, d_sys, lds_per_path);
