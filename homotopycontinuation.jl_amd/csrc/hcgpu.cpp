@@ -288,12 +288,18 @@ static int hcg_generate_impl(const hcg_homotopy_desc* h, char* buf, size_t bufsz
     return HCG_OK;
 }
 
-// Default register budget of the tracker kernels: waves per SIMD they are built for.  A loaded
-// kernel waits for the traffic of its lanes' private state, which a second wave per SIMD doubles
-// and half the registers per lane make larger still.  One against two waves, measured: parameter
+// Default register budget of the tracker kernels: waves per SIMD they are built for.  Up to n = 10 a
+// solve's matrix stays in the 512 registers of one wave per SIMD, and a loaded kernel waits for the traffic
+// of its lanes' private state, which a second wave doubles.  One against two waves, measured: parameter
 // batch n = 10, 1,024 paths plain 48.5 / 50.5 ms, 61,777 plain 153.7 / 163.7, 262,144 learned 294.6 /
-// 307.8; dense n = 8, 6,561 paths 152.6 / 251.2.
-static const int kDefaultWavesPerEU = 1;
+// 307.8; dense n = 8, 6,561 paths 152.6 / 251.2.  Past n = 10 the matrix does not fit and the long
+// straight-line evaluations need a second wave to issue beside: shared-factor cubics n = 12, learned, 30,000
+// paths 317.7 / 341.4 ms, 131,072 paths 739.8 / 640.7, 531,441 paths 2,314.9 / 1,907.1.
+static int default_waves(const hcg_homotopy_desc* const* hs, int32_t nsys) {
+    int n = 0;
+    for (int s = 0; s < nsys; s++) n = std::max<int>(n, hs[s]->n);
+    return n <= 10 ? 1 : 2;
+}
 
 static int build_source(const hcg_homotopy_desc* const* hs, int32_t nsys, int32_t multi, const hcg_build_options* bo,
                         std::string* src, std::vector<hcg::Flops>* fl) {
@@ -301,7 +307,7 @@ static int build_source(const hcg_homotopy_desc* const* hs, int32_t nsys, int32_
     for (int s = 0; s < nsys; s++)
         if (!hs[s]) return fail(HCG_ERR_INVALID_ARGUMENT, "homotopy %d is NULL", s);
     if (nsys > 1 && !multi) return fail(HCG_ERR_INVALID_ARGUMENT, "several homotopies need a multi-system program");
-    int w = bo && bo->waves_per_eu ? bo->waves_per_eu : kDefaultWavesPerEU;
+    int w = bo && bo->waves_per_eu ? bo->waves_per_eu : default_waves(hs, nsys);
     if (w != 1 && w != 2 && w != 4 && w != 8) return fail(HCG_ERR_INVALID_ARGUMENT, "waves_per_eu must be 1, 2, 4 or 8");
     std::string body, err;
     fl->assign(nsys, hcg::Flops());
@@ -368,7 +374,7 @@ static int hcg_program_create_ex_impl(hcg_ctx* ctx, const hcg_homotopy_desc* con
     std::vector<hcg::Flops> fl;
     int rc = build_source(hs, nsys, multi, bo, &p->source, &fl);
     if (rc) { delete p; return rc; }
-    p->waves_per_eu = bo && bo->waves_per_eu ? bo->waves_per_eu : kDefaultWavesPerEU;
+    p->waves_per_eu = bo && bo->waves_per_eu ? bo->waves_per_eu : default_waves(hs, nsys);
     if (multi) {
         p->nsys = nsys;
         for (int s = 0; s < nsys; s++) {

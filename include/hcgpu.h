@@ -171,7 +171,8 @@ int hcg_compile_multi_only(const hcg_homotopy_desc* const* hs, int32_t nsys, siz
 
 /* Build choices of a program (no counterpart in the reference; picked by the autotuner).
  * waves_per_eu: waves per SIMD the tracker kernel is compiled for, i.e. a register budget
- * of 512 / waves_per_eu per lane (1, 2, 4 or 8; 0 = the library default, 1; per-lane layout).
+ * of 512 / waves_per_eu per lane (1, 2, 4 or 8; 0 = the library default, 1 up to n = 10 and
+ * 2 past it; per-lane layout).
  * layout: HCG_LAYOUT_LANE (one path per lane, the tapes compiled with hipRTC) or
  * HCG_LAYOUT_GROUP (one path per group of 16 lanes, 32 lanes for 17 to 24 variables, each
  * lane holding one row of the Jacobian and one entry of every vector in registers; the tapes
