@@ -69,6 +69,47 @@ def sparse_param_system(n: int = 10, nterms: int = 20, nparams: int = 16, seed: 
     return System(polys, n, nparams)
 
 
+def sparse_solution(F: System, rng):
+    """(x0, p0) with F(x0; p0) = 0 for a system whose coefficients are affine in its parameters: a
+    random point and the least-norm parameters, the solution of a linear system."""
+    n, m = F.nvars, F.nparams
+    x0 = cgauss(rng, n)
+    A, b = np.zeros((n, m), dtype=complex), np.zeros(n, dtype=complex)
+    for i, f in enumerate(F.polys):
+        for e, c in f.terms.items():
+            v = complex(c) * np.prod(x0 ** np.array(e[:n]))
+            if any(e[n:]):
+                A[i, e[n:].index(1)] += v
+            else:
+                b[i] -= v
+    return x0, np.linalg.lstsq(A, b, rcond=None)[0]
+
+
+def solve_size_homotopy(n: int):
+    """(H, x0): a parameter homotopy of n sparse quadrics with one start solution x0 and nine targets,
+    small enough for a check against a CPU tracker at every n."""
+    from .homotopies import ParameterHomotopy
+    F = sparse_param_system(n, 3 if n == 1 else 4, n + 2, seed=n)
+    rng = np.random.default_rng(n)
+    x0, p0 = sparse_solution(F, rng)
+    return ParameterHomotopy(F, p0, p0 + 0.3 * cgauss(rng, 9, n + 2), lift_affine=True), x0
+
+
+def parameter_product_system() -> System:
+    """Three quadrics whose coefficients are products of four parameters, raw parameters and
+    constants, some shared by rows."""
+    (x, y, z), p = variables(3, 4)
+    rng = np.random.default_rng(9)
+    mons = [x * y, y * z, x * z, x, y, z]
+    rows = []
+    for i, sq in enumerate((x**2, y**2, z**2)):
+        f = sq + p[i] * mons[i] - 1
+        for k, m in enumerate(mons):
+            f = f + (complex(cgauss(rng)) * p[k % 4] * p[(k + i) % 4] + complex(cgauss(rng)) * p[(k + 1) % 4]) * m
+        rows.append(f)
+    return System(rows, 3, 4)
+
+
 def shared_factor_system(n: int, seed: int = 0) -> System:
     rng = np.random.default_rng(seed)
     xs, _ = variables(n)

@@ -5,9 +5,8 @@ import pytest
 
 import oracle
 from hcgpu.certify import parameter_boxes
-from hcgpu.configs import cgauss, sparse_param_system
+from hcgpu.configs import cgauss, parameter_product_system, sparse_param_system
 from hcgpu.homotopies import _SysTapes
-from hcgpu.polys import System, variables
 
 pytestmark = pytest.mark.gpu
 
@@ -15,17 +14,7 @@ pytestmark = pytest.mark.gpu
 def system(name):
     if name == "affine3":  # 72 coefficient operations, affine in four parameters
         return sparse_param_system(3, 6, 4, seed=7)
-    # coefficients that are products of parameters, raw parameters and constants, some shared by rows
-    (x, y, z), p = variables(3, 4)
-    rng = np.random.default_rng(9)
-    mons = [x * y, y * z, x * z, x, y, z]
-    rows = []
-    for i, sq in enumerate((x**2, y**2, z**2)):
-        f = sq + p[i] * mons[i] - 1
-        for k, m in enumerate(mons):
-            f = f + (complex(cgauss(rng)) * p[k % 4] * p[(k + i) % 4] + complex(cgauss(rng)) * p[(k + 1) % 4]) * m
-        rows.append(f)
-    return System(rows, 3, 4)
+    return parameter_product_system()
 
 
 def _zeros(F, q, rng):
