@@ -232,8 +232,10 @@ __device__ __noinline__ void cert_refine_dd(cdd* xd, const cplx* C, const double
 #define CERT_IJ (14 * HCG_CERT_NCE)
 #define CERT_BJ (14 * HCG_CERT_NCE + 4 * HCG_CERT_NCJ)
 #define CERT_COEF (14 * HCG_CERT_NCE + 10 * HCG_CERT_NCJ)
-// One lane per coefficient and parameter vector.
-extern "C" __global__ void __launch_bounds__(64) hcg_cert_coef_kernel(hcg_cert_kargs a) {
+// One lane per coefficient and parameter vector.  The same register budget as the certifier below: they
+// share the interpreters, whose code takes the largest budget among their callers (without it the
+// certifier was built with 164 registers, three waves per SIMD).
+extern "C" __global__ void __launch_bounds__(64, 4) hcg_cert_coef_kernel(hcg_cert_kargs a) {
     const int per = HCG_CERT_NCE + HCG_CERT_NCJ;
     const long t = (long)blockIdx.x * 64 + threadIdx.x;
     if (t >= (long)(a.g1 - a.g0) * per) return;
