@@ -430,8 +430,9 @@ static void emit_tables(std::ostringstream& os, const std::string& fname, const 
     os << "};\n";
 }
 
+// table: the tape's parameters are the entries of a double-double table (DDTab)
 static void gen_dd_interp(std::ostringstream& os, const hcg_tape* tp, const std::string& fname, int n, ParamMode pm,
-                          const double* fixed, long* flops) {
+                          const double* fixed, long* flops, bool table = false) {
     std::vector<std::pair<int, int>> outs;
     for (int i = 0; i < tp->nu; i++) outs.push_back({tp->u_assign[2 * i] - 1, tp->u_assign[2 * i + 1]});
     const InterpPlan P = plan_interp(tp, outs, n, pm, fixed, 1 << 24);
@@ -441,10 +442,12 @@ static void gen_dd_interp(std::ostringstream& os, const hcg_tape* tp, const std:
     const auto& out_operand = P.out_operand;
     emit_tables(os, fname, P);
     os << "__device__ __noinline__ void " << fname << "(const cdd* __restrict__ x, ";
-    if (pm == PM_DYNAMIC) os << "const double* __restrict__ pp, const double* __restrict__ pq, cplx pt, ";
+    if (table) os << "const double* __restrict__ pc, ";
+    else if (pm == PM_DYNAMIC) os << "const double* __restrict__ pp, const double* __restrict__ pq, cplx pt, ";
     os << "cdd* __restrict__ u) {\n";
     os << "  cdd R[" << std::max(nreg, 1) << "];\n";
-    os << "  DDPar P; P.p = " << (pm == PM_DYNAMIC ? "(hcg_gld*)pp" : "nullptr") << "; P.q = " << (pm == PM_DYNAMIC ? "(hcg_gld*)pq" : "nullptr")
+    if (table) os << "  DDTab P; P.c = (hcg_gld*)pc;\n";
+    else os << "  DDPar P; P.p = " << (pm == PM_DYNAMIC ? "(hcg_gld*)pp" : "nullptr") << "; P.q = " << (pm == PM_DYNAMIC ? "(hcg_gld*)pq" : "nullptr")
        << "; P.t = " << (pm == PM_DYNAMIC ? "pt" : "mkc(0.0, 0.0)") << ";\n";
     for (auto& ld : loads) os << "  R[" << ld.first << "] = x[" << (ld.second - tp->nparams) << "];\n";
     os << "  dd_interpret(" << fname << "_code, " << ninstr << ", " << fname << "_const, R, P);\n";
@@ -1075,7 +1078,7 @@ static void emit_cones(std::ostringstream& os, const hcg_tape* tp, const std::st
     const std::string nr = std::to_string(std::max(S.nreg, 1));
     os << "__device__ __noinline__ void " << fname << "_coef(int c, const double* P, const double* IP, const double* BP, double* D, double* I, double* B) {\n";
     if (dd) {
-        os << "  { cdd R[" << nr << "]; DDPar Q; Q.p = (hcg_gld*)P; Q.q = (hcg_gld*)P; Q.t = mkc(0.0, 0.0);\n    dd_interpret(" << args << ", R, Q);\n"
+        os << "  { cdd R[" << nr << "]; DDPoint Q; Q.p = (hcg_gld*)P;\n    dd_interpret(" << args << ", R, Q);\n"
            << "    const cdd v = dd_fetch(" << fname << "_cone_const, R, Q, " << fname << "_out[c]);\n"
            << "    double* o = D + 4 * c; o[0] = v.re.hi; o[1] = v.re.lo; o[2] = v.im.hi; o[3] = v.im.lo; }\n";
     }
@@ -1110,7 +1113,7 @@ bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::
     const hcg_tape* te = split ? &se.main : F->eval;
     const hcg_tape* tj = split ? &sj.main : F->eval_jac;
     os << "#define HCG_CERT_NCE " << (split ? se.main.nparams : 0) << "\n#define HCG_CERT_NCJ " << (split ? sj.main.nparams : 0) << "\n";
-    gen_dd_interp(os, te, "certF_eval_dd", n, pm, fixed, &f);
+    gen_dd_interp(os, te, "certF_eval_dd", n, pm, fixed, &f, split);
     gen_cert_interp(os, te, "cert_ieval", false, n, pm, fixed, false);
     gen_cert_interp(os, tj, "cert_ijac", true, n, pm, fixed, false);
     gen_cert_interp(os, te, "cert_beval", false, n, pm, fixed, true);
@@ -1122,7 +1125,7 @@ bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::
     const std::string pa = pm == PM_DYNAMIC ? "P, P, mkc(0.0, 0.0), " : "";
     os << "HD void cert_eval_jac(const cplx* x, const double* P, cplx* u, cplx* U) { certF_eval_jac(x, " << pa << "u, U); }\n";
     os << "HD void cert_eval_dd(const cdd* x, const double* P, cdd* u) { certF_eval_dd(x, "
-       << (split ? "P, nullptr, mkc(0.0, 0.0), " : pa) << "u); }\n";
+       << (split ? "P, " : pa) << "u); }\n";
     os << "#include \"hcg_certify.h\"\n";
     *src = os.str();
     return true;

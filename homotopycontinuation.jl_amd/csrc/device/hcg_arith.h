@@ -465,17 +465,28 @@ struct DDPar {
     hcg_gld* q;
     cplx t;
 };
-HD cdd dd_fetch(const double* K, const cdd* R, const DDPar& P, int e) {
-#ifdef HCG_P_PER_LANE
-    if (e >= DD_PBASE && !P.q) {  // a certifier's coefficient tables hold double-double values
-        hcg_gld* c = P.p + 4 * (e - DD_PBASE);
-        return mkcdd(mkdd(c[0], c[1]), mkdd(c[2], c[3]));
-    }
-#endif
-    if (e >= DD_PBASE) return cdd_from(par_lerp(P.t, P.p, P.q, e - DD_PBASE));
+HD cdd dd_param(const DDPar& P, int k) { return cdd_from(par_lerp(P.t, P.p, P.q, k)); }
+// The certifier's other two kinds: the parameters at t = 0 (the programs of its coefficients), and a
+// coefficient table of double-double values.  Types of their own, so that dd_interpret is
+// compiled for each caller: with one caller the compiler knows its tables' addresses (with the
+// parameter-only programs as a second caller of the whole tapes' instance a Newton iteration
+// of the certifier took 10 to 20% longer).
+struct DDPoint {
+    hcg_gld* p;
+};
+HD cdd dd_param(const DDPoint& P, int k) { return cdd_from(par_lerp(mkc(0.0, 0.0), P.p, P.p, k)); }
+struct DDTab {
+    hcg_gld* c;
+};
+HD cdd dd_param(const DDTab& P, int k) {
+    hcg_gld* c = P.c + 4 * k;
+    return mkcdd(mkdd(c[0], c[1]), mkdd(c[2], c[3]));
+}
+template <class PAR> HD cdd dd_fetch(const double* K, const cdd* R, const PAR& P, int e) {
+    if (e >= DD_PBASE) return dd_param(P, e - DD_PBASE);
     return e >= 0 ? R[e] : cdd_from(mkc(K[2 * (-e - 1)], K[2 * (-e - 1) + 1]));
 }
-__device__ __noinline__ void dd_interpret(const int* code, int ninstr, const double* K, cdd* R, DDPar P) {
+template <class PAR> __device__ __noinline__ void dd_interpret(const int* code, int ninstr, const double* K, cdd* R, PAR P) {
     for (int i = 0; i < ninstr; i++) {
         const int* I = code + 6 * i;
         const int op = I[0];
