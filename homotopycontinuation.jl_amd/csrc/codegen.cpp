@@ -961,6 +961,7 @@ struct SplitTape {
     hcg_tape main;
     std::vector<InterpPlan> cones;
     int nreg = 0;  // registers of the largest cone
+    long saved = 0, cone_ops = 0;  // operations that leave the tape; operations of all cones
 };
 // Below this many parameter-only operations the tape stays whole.
 static const int kSplitMin = 32;
@@ -993,6 +994,7 @@ static bool split_tape(const hcg_tape* tp, const std::vector<std::pair<int, int>
         def_of[I[5]] = first + i;
     }
     if (npo < kSplitMin) return false;
+    S->saved = npo;
     std::vector<int> coef(first + ninstr, -1), order;
     auto need = [&](int d) { if (d >= 0 && ponly[d] && coef[d] < 0) { coef[d] = (int)order.size(); order.push_back(d); } };
     for (int i = 0; i < ninstr; i++)
@@ -1032,7 +1034,6 @@ static bool split_tape(const hcg_tape* tp, const std::vector<std::pair<int, int>
     S->main.u_assign = S->u_assign.data();
     S->main.U_assign = S->U_assign.data();
     // the cones, each with the instructions it reaches; shared ones are repeated
-    long total = 0;
     for (int d : order) {
         std::vector<char> use(first + ninstr, 0);
         use[d] = 1;
@@ -1054,8 +1055,8 @@ static bool split_tape(const hcg_tape* tp, const std::vector<std::pair<int, int>
         const int os = d < np ? tp->params_first + d : tp->tape_space + 1 + d - first;
         S->cones.push_back(plan_interp(&c, {{0, os}}, 1, PM_DYNAMIC, nullptr, 1 << 24));
         S->nreg = std::max(S->nreg, S->cones.back().nreg);
-        total += c.ninstr;
-        if (total > 4L * ninstr + 64) return false;  // heavily shared: the cones would repeat too much
+        S->cone_ops += c.ninstr;
+        if (S->cone_ops > 4L * ninstr + 64) return false;  // heavily shared: the cones would repeat too much
     }
     return true;
 }
@@ -1098,7 +1099,7 @@ bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::
     const ParamMode pm = np == 0 ? PM_NONE : (F->fixed_params ? PM_FIXED : PM_DYNAMIC);
     const double* fixed = F->fixed_params;
     std::ostringstream os;
-    os << "// generated by hcgpu codegen (certifier)\n#define HCG_P_PER_LANE\n#include \"hcg_arith.h\"\n#include \"hcg_interval.h\"\n";
+    os << "// generated by hcgpu codegen (certifier)\n#define HCG_P_PER_LANE\n#include \"hcg_arith.h\"\n#include \"hcg_interval.h\"\n#include \"hcg_cert_kargs.h\"\n";
     os << "#define HCG_N " << n << "\n#define HCG_NPAR " << (pm == PM_DYNAMIC ? np : 0) << "\n";
     long f;
     gen_eval(os, F->eval_jac, "certF_eval_jac", true, false, n, pm, fixed, &f);
@@ -1110,23 +1111,32 @@ bool generate_certify_source(const hcg_system* F, int n, std::string* src, std::
     for (int i = 0; i < F->eval->nu; i++) oe.push_back({F->eval->u_assign[2 * i] - 1, F->eval->u_assign[2 * i + 1]});
     for (int i = 0; i < F->eval_jac->nU; i++) oj.push_back({F->eval_jac->U_assign[2 * i] - 1, F->eval_jac->U_assign[2 * i + 1]});
     const bool split = pm == PM_DYNAMIC && split_tape(F->eval, oe, &se) && split_tape(F->eval_jac, oj, &sj);
-    const hcg_tape* te = split ? &se.main : F->eval;
-    const hcg_tape* tj = split ? &sj.main : F->eval_jac;
-    os << "#define HCG_CERT_NCE " << (split ? se.main.nparams : 0) << "\n#define HCG_CERT_NCJ " << (split ? sj.main.nparams : 0) << "\n";
-    gen_dd_interp(os, te, "certF_eval_dd", n, pm, fixed, &f, split);
-    gen_cert_interp(os, te, "cert_ieval", false, n, pm, fixed, false);
-    gen_cert_interp(os, tj, "cert_ijac", true, n, pm, fixed, false);
-    gen_cert_interp(os, te, "cert_beval", false, n, pm, fixed, true);
-    gen_cert_interp(os, tj, "cert_bjac", true, n, pm, fixed, true);
-    if (split) {
-        emit_cones(os, F->eval, "certE", se, true);
-        emit_cones(os, F->eval_jac, "certJ", sj, false);
-    }
     const std::string pa = pm == PM_DYNAMIC ? "P, P, mkc(0.0, 0.0), " : "";
     os << "HD void cert_eval_jac(const cplx* x, const double* P, cplx* u, cplx* U) { certF_eval_jac(x, " << pa << "u, U); }\n";
-    os << "HD void cert_eval_dd(const cdd* x, const double* P, cdd* u) { certF_eval_dd(x, "
-       << (split ? "P, " : pa) << "u); }\n";
-    os << "#include \"hcg_certify.h\"\n";
+    // what hcg_certify.h evaluates besides, on the tapes te and tj
+    auto kernel = [&](const hcg_tape* te, const hcg_tape* tj, bool tables, const std::string& name) {
+        gen_dd_interp(os, te, "certF_eval_dd", n, pm, fixed, &f, tables);
+        gen_cert_interp(os, te, "cert_ieval", false, n, pm, fixed, false);
+        gen_cert_interp(os, tj, "cert_ijac", true, n, pm, fixed, false);
+        gen_cert_interp(os, te, "cert_beval", false, n, pm, fixed, true);
+        gen_cert_interp(os, tj, "cert_bjac", true, n, pm, fixed, true);
+        os << "HD void cert_eval_dd(const cdd* x, const double* P, cdd* u) { certF_eval_dd(x, " << (tables ? "P, " : pa) << "u); }\n";
+        os << "#define HCG_CERT_KERNEL " << name << "\n#include \"hcg_certify.h\"\n#undef HCG_CERT_KERNEL\n";
+    };
+    if (split) {
+        os << "#define HCG_CERT_NCE " << se.main.nparams << "\n#define HCG_CERT_NCJ " << sj.main.nparams << "\n";
+        os << "#define HCG_CERT_SAVED_OPS " << se.saved + sj.saved << "\n#define HCG_CERT_CONE_OPS " << se.cone_ops + sj.cone_ops << "\n";
+        emit_cones(os, F->eval, "certE", se, true);
+        emit_cones(os, F->eval_jac, "certJ", sj, false);
+        os << "namespace tables {\n";
+        kernel(&se.main, &sj.main, true, "hcg_certify_kernel");
+        os << "}  // namespace tables\n#undef HCG_CERT_NCE\n#undef HCG_CERT_NCJ\nnamespace whole {\n";
+        kernel(F->eval, F->eval_jac, false, "hcg_certify_whole_kernel");
+        os << "}  // namespace whole\n";
+    } else {
+        os << "#define HCG_CERT_NCE 0\n";
+        kernel(F->eval, F->eval_jac, false, "hcg_certify_kernel");
+    }
     *src = os.str();
     return true;
 }

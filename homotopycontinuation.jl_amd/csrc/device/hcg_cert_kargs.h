@@ -12,8 +12,8 @@ typedef struct hcg_cert_kargs {
     const double* params;         // per group: nparams complex (point), or NULL
     const double* params_ival;    // per group: nparams * 4 (re lo, re hi, im lo, im hi), or NULL
     const double* params_ball;    // per group: nparams * 6 (re hi, re lo, re rad, im hi, im lo, im rad), or NULL
-    double* coef;                 // per group of this launch: coefficient tables (split tapes), or NULL
-    int32_t g0, g1;               // groups of this launch: candidates of other groups are left alone
+    double* coef;                 // per group: coefficient tables (split tapes), or NULL
+    int64_t ngroups;
     const int32_t* group_of;      // nsol group indices (checked by the host) or NULL (group 0)
     hcg_certificate* out;         // nsol records
     double* box1;                 // nsol * n * 4: the certified box x₁

@@ -27,8 +27,9 @@
 // hcg_cert_coef_kernel.
 // P is the parameter point (HCG_NPAR complex), IP its box (HCG_NPAR × 4 doubles) and BP
 // its double-double ball (HCG_NPAR × 6 doubles).
-#pragma once
-#include "hcg_cert_kargs.h"
+// No include guard on purpose: where the tapes are split the source includes it twice, in
+// two namespaces: once with the tables and once with the whole tapes (HCG_CERT_NCE undefined), for
+// launches with many parameter vectors.  HCG_CERT_KERNEL is the certifier kernel's name.
 
 #define CN HCG_N
 #define CAT(A, i, j) A[(i) + (j) * CN]
@@ -238,13 +239,13 @@ __device__ __noinline__ void cert_refine_dd(cdd* xd, const cplx* C, const double
 extern "C" __global__ void __launch_bounds__(64, 4) hcg_cert_coef_kernel(hcg_cert_kargs a) {
     const int per = HCG_CERT_NCE + HCG_CERT_NCJ;
     const long t = (long)blockIdx.x * 64 + threadIdx.x;
-    if (t >= (long)(a.g1 - a.g0) * per) return;
-    const long s = t / per, g = a.g0 + s;
+    if (t >= a.ngroups * per) return;
+    const long g = t / per;
     const int c = (int)(t % per);
     const double* P = a.params + 2 * HCG_NPAR * g;
     const double* IP = a.params_ival + 4 * HCG_NPAR * g;
     const double* BP = a.params_ball + 6 * HCG_NPAR * g;
-    double* T = a.coef + CERT_COEF * s;
+    double* T = a.coef + CERT_COEF * g;
     if (c < HCG_CERT_NCE) certE_coef(c, P, IP, BP, T, T + CERT_IE, T + CERT_BE);
     else certJ_coef(c - HCG_CERT_NCE, P, IP, BP, T, T + CERT_IJ, T + CERT_BJ);
 }
@@ -253,7 +254,7 @@ extern "C" __global__ void __launch_bounds__(64, 4) hcg_cert_coef_kernel(hcg_cer
 // Four waves per SIMD (128 registers per lane): the kernel is latency-bound on its private
 // memory, and occupancy beats registers here.  Measured on 262,144 candidates at n = 10 with whole tapes:
 // 176 ms at one wave per SIMD, 109 ms at two, 81 ms at four, 127 ms at eight.
-extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_kargs a) {
+extern "C" __global__ void __launch_bounds__(64, 4) HCG_CERT_KERNEL(hcg_cert_kargs a) {
     const long k = (long)blockIdx.x * 64 + threadIdx.x;
     if (k >= a.nsol) return;
     const int g = a.group_of ? a.group_of[k] : 0;
@@ -262,8 +263,7 @@ extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_
     const double* BP = a.params_ball ? a.params_ball + 6 * HCG_NPAR * g : nullptr;
     // what the double-double, interval and ball evaluations read: the parameters, or coefficient tables
 #if HCG_CERT_NCE > 0
-    if (g < a.g0 || g >= a.g1) return;
-    const double* T = a.coef + (long)CERT_COEF * (g - a.g0);
+    const double* T = a.coef + (long)CERT_COEF * g;
     const double *PD = T, *IE = T + CERT_IE, *IJ = T + CERT_IJ, *BE = T + CERT_BE, *BJ = T + CERT_BJ;
 #else
     const double *PD = P, *IE = IP, *IJ = IP, *BE = BP, *BJ = BP;
@@ -358,3 +358,10 @@ extern "C" __global__ void __launch_bounds__(64, 4) hcg_certify_kernel(hcg_cert_
     c.inflation = o.inflation;
     a.out[k] = c;
 }
+#undef CN
+#undef CAT
+#undef CERT_IE
+#undef CERT_BE
+#undef CERT_IJ
+#undef CERT_BJ
+#undef CERT_COEF

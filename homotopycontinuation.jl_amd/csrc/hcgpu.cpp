@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "hcg_codegen.h"
+#include "hcg_launch_rules.h"
 #include "hcg_group_launch.h"
 #include "hcg_mlp.h"
 #include "hcg_noalloc.h"
@@ -81,8 +82,9 @@ struct hcg_program {
     // certifier programs (hcg_certifier_create): the kernel is hcg_certify_kernel
     bool certifier = false;
     int cert_npar = 0;  // parameters given per hcg_certify call (0 when fixed or absent)
-    hipFunction_t coef_kernel = nullptr;  // split tapes: fills the coefficient tables
-    long coef_per_group = 0, coef_doubles = 0;  // coefficients and table size of one parameter vector
+    hipFunction_t coef_kernel = nullptr;   // split tapes: fills the coefficient tables
+    hipFunction_t whole_kernel = nullptr;  // split tapes: the certifier without tables
+    hcg::CertSplit split = {0, 0, 0, 0};
     // lane-group layout (hcg_build_options.layout = 1): slot programs for the precompiled kernel
     hcg::GroupPrograms* group = nullptr;
 };
@@ -1114,23 +1116,21 @@ static int hcg_certifier_create_impl(hcg_ctx* ctx, const hcg_system* F, int32_t 
     if (e != hipSuccess) { delete p; return fail(HCG_ERR_HIP, "hipModuleLoadData: %s", hipGetErrorString(e)); }
     e = hipModuleGetFunction(&p->kernel, p->module, "hcg_certify_kernel");
     if (e != hipSuccess) { hipModuleUnload(p->module); delete p; return fail(HCG_ERR_HIP, "hipModuleGetFunction: %s", hipGetErrorString(e)); }
-    long nce = 0, ncj = 0;  // as the generated source states them
-    for (auto& kv : {std::make_pair("#define HCG_CERT_NCE ", &nce), std::make_pair("#define HCG_CERT_NCJ ", &ncj)}) {
-        const size_t at = p->source.find(kv.first);
-        if (at != std::string::npos) *kv.second = std::atol(p->source.c_str() + at + std::strlen(kv.first));
-    }
+    auto stated = [&](const char* macro) -> long {  // as the generated source states it
+        const std::string def = std::string("#define ") + macro + " ";
+        const size_t at = p->source.find(def);
+        return at == std::string::npos ? 0 : std::atol(p->source.c_str() + at + def.size());
+    };
+    const long nce = stated("HCG_CERT_NCE"), ncj = stated("HCG_CERT_NCJ");
     if (nce > 0) {
-        p->coef_per_group = nce + ncj;
-        p->coef_doubles = 14 * nce + 10 * ncj;
+        p->split = {nce + ncj, 14 * nce + 10 * ncj, stated("HCG_CERT_SAVED_OPS"), stated("HCG_CERT_CONE_OPS")};
         e = hipModuleGetFunction(&p->coef_kernel, p->module, "hcg_cert_coef_kernel");
+        if (e == hipSuccess) e = hipModuleGetFunction(&p->whole_kernel, p->module, "hcg_certify_whole_kernel");
         if (e != hipSuccess) { hipModuleUnload(p->module); delete p; return fail(HCG_ERR_HIP, "hipModuleGetFunction: %s", hipGetErrorString(e)); }
     }
     *out = p;
     return HCG_OK;
 }
-
-// Most bytes of coefficient tables held at once; more parameter vectors take several launches.
-static const size_t kCoefBytes = (size_t)1 << 30;
 
 static int hcg_certify_impl(hcg_ctx* ctx, const hcg_program* prog, int32_t nsol, const double* cand,
                             int32_t ngroups, const double* params, const double* params_ival,
@@ -1212,23 +1212,22 @@ static int hcg_certify_impl(hcg_ctx* ctx, const hcg_program* prog, int32_t nsol,
     const unsigned grid = (unsigned)(((long)nsol + 63) / 64);  // one lane per candidate, 64 per workgroup
     void* args[] = {&ka};
     DevBuf d_coef;
-    long chunk = ngroups;  // parameter vectors per launch
-    if (prog->coef_kernel) {
-        const size_t one = sizeof(double) * (size_t)prog->coef_doubles;
-        chunk = std::max<long>(1, std::min<long>(ngroups, (long)(kCoefBytes / one)));
-        HIPCHK(hipMalloc(&d_coef.p, one * (size_t)chunk));
+    if (prog->coef_kernel && hcg::certify_with_tables(nsol, ngroups, prog->split)) {
+        // no room for the tables: the whole tapes need none
+        if (hipMalloc(&d_coef.p, sizeof(double) * (size_t)prog->split.doubles * ngroups) != hipSuccess) {
+            (void)hipGetLastError();
+            d_coef.p = nullptr;
+        }
         ka.coef = (double*)d_coef.p;
+        ka.ngroups = ngroups;
     }
     HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
-    for (long g = 0; g == 0 || g < ngroups; g += std::max<long>(chunk, 1)) {
-        ka.g0 = (int32_t)g;
-        ka.g1 = (int32_t)std::min<long>(ngroups, g + chunk);
-        if (prog->coef_kernel) {
-            const unsigned cg = (unsigned)(((long)(ka.g1 - ka.g0) * prog->coef_per_group + 63) / 64);
-            HIPCHK(hipModuleLaunchKernel(prog->coef_kernel, cg, 1, 1, 64, 1, 1, 0, ctx->stream, args, nullptr));
-        }
-        HIPCHK(hipModuleLaunchKernel(prog->kernel, grid, 1, 1, 64, 1, 1, 0, ctx->stream, args, nullptr));
+    if (ka.coef) {
+        const unsigned cg = (unsigned)(((long)ngroups * prog->split.coefs + 63) / 64);
+        HIPCHK(hipModuleLaunchKernel(prog->coef_kernel, cg, 1, 1, 64, 1, 1, 0, ctx->stream, args, nullptr));
     }
+    hipFunction_t kernel = prog->coef_kernel && !ka.coef ? prog->whole_kernel : prog->kernel;
+    HIPCHK(hipModuleLaunchKernel(kernel, grid, 1, 1, 64, 1, 1, 0, ctx->stream, args, nullptr));
     HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
     HIPCHK(hipMemcpyAsync(out, d_out.p, sizeof(hcg_certificate) * nsol, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipMemcpyAsync(box1, d_b1.p, zb, hipMemcpyDeviceToHost, ctx->stream));

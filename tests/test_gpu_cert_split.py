@@ -63,3 +63,24 @@ def test_split_equals_whole(gpu_ctx, name, ngroups):
         np.testing.assert_array_equal(g.box0, o.box0)
         np.testing.assert_array_equal(g.refined, o.refined)
     assert g.certified.any()
+
+
+@pytest.mark.parametrize("name,nsol,ngroups", [("affine3", 12014, 12014), ("affine3", 12015, 12015), ("products3", 4372, 4372),
+                                               ("products3", 4373, 4373), ("products3", 9000, 4661), ("products3", 9000, 4662)])
+def test_tables_or_whole_tapes(gpu_ctx, name, nsol, ngroups):
+    """The largest number of parameter vectors that takes tables, and the smallest that takes whole
+    tapes, with groups out of order; random points, about half of which converge to zeros."""
+    F = system(name)
+    rng = np.random.default_rng(nsol + ngroups)
+    Q, X = cgauss(rng, ngroups, 4), cgauss(rng, nsol, 3)
+    G = rng.permutation(np.arange(nsol, dtype=np.int32) % ngroups)
+    g = gpu_ctx.certifier(F).certify(X, Q, real_system=False, group_of=G)
+    enc = [parameter_boxes(list(q)) for q in Q]
+    P, I, B = (np.stack([e[k] for e in enc]) for k in range(3))
+    tapes = _SysTapes(F)
+    o = oracle.certify(tapes.struct(), 3, X, P, I, B, True, True, False, 16, group_of=G)
+    for f in ("certified", "newton_iters", "prec", "contraction", "inflation"):
+        np.testing.assert_array_equal(getattr(g, f), getattr(o, f), err_msg=f)
+    np.testing.assert_array_equal(g.box1, o.box1)
+    np.testing.assert_array_equal(g.refined, o.refined)
+    assert 0 < g.certified.sum() < nsol
