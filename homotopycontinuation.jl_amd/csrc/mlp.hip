@@ -259,25 +259,16 @@ __global__ void fill_zero(float* p, int n) {
     } while (0)
 
 int ensure(hcg::MlpWork* w, long n, std::string* err) {
-    if (!w->params) {
-        CK(hipMalloc(&w->params, sizeof(float) * NP));
-        CK(hipMalloc(&w->grad, sizeof(float) * NP));
-        CK(hipMalloc(&w->adam_m, sizeof(float) * NP));
-        CK(hipMalloc(&w->adam_v, sizeof(float) * NP));
-        CK(hipMalloc(&w->loss, sizeof(float)));
-        CK(hipMalloc(&w->part, sizeof(float) * PS * kMaxBlocks));
-    }
-    if (n > w->cap) {
-        hipFree(w->x); hipFree(w->y); hipFree(w->w); hipFree(w->pred); hipFree(w->perm);
-        w->x = w->y = w->w = w->pred = nullptr; w->perm = nullptr;
-        CK(hipMalloc(&w->x, sizeof(float) * IN * n));
-        CK(hipMalloc(&w->y, sizeof(float) * OUT * n));
-        CK(hipMalloc(&w->w, sizeof(float) * OUT * n));
-        CK(hipMalloc(&w->pred, sizeof(float) * OUT * n));
-        CK(hipMalloc(&w->perm, sizeof(int32_t) * n));
-        w->cap = n;
-    }
-    return HCG_OK;
+    auto alloc = [&](size_t bytes) -> void* {
+        void* p = nullptr;
+        const hipError_t e = hipMalloc(&p, bytes);
+        if (e == hipSuccess) return p;
+        (void)hipGetLastError();
+        *err = std::string("hipMalloc of the training workspace: ") + hipGetErrorString(e);
+        return nullptr;
+    };
+    const bool ok = hcg::mlp_work_ensure(w, n, IN, OUT, NP, (size_t)PS * kMaxBlocks, alloc, [](void* p) { (void)hipFree(p); });
+    return ok ? HCG_OK : HCG_ERR_HIP;
 }
 
 int tile_blocks(int cnt) { return std::min((cnt + R - 1) / R, kMaxBlocks); }
