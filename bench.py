@@ -52,7 +52,7 @@ def measured_traffic(workload: str):
     return round((t["fetch_kib"] * t["fetch_scale"] + t["write_kib"] * t["write_scale"]) * 1024.0)
 
 
-def roofline(flops, kernel_ms, workload, kernel="hcg_track_kernel", info=None, grid_waves=None):
+def roofline(flops, kernel_ms, workload, kernel="hcg_track_kernel", info=None):
     """The tracker kernel against its algorithmic roof, MI355X's FP64 vector peak (no MFMA is
     used: the linear algebra is a few percent of a step's flops at these sizes), with what the
     profiles measured beside it: HBM traffic per launch (the bound the per-lane kernel actually
@@ -84,25 +84,13 @@ def roofline(flops, kernel_ms, workload, kernel="hcg_track_kernel", info=None, g
             "profile": prof.get("counters_source")}
     if info is not None:
         occ = dict(info)
-        if grid_waves is not None:
-            occ["grid_waves"] = int(grid_waves)
-            occ["resident_waves_per_simd"] = round(min(grid_waves, 4 * info["cus"] * info["waves_per_simd_built"])
-                                                   / (4 * info["cus"]), 3)
+        occ["grid_waves"] = occ.pop("waves")
+        occ["resident_waves_per_simd"] = round(min(occ["grid_waves"], 4 * info["cus"] * info["waves_per_simd_built"])
+                                               / (4 * info["cus"]), 3)
         if "mean_occupancy_per_cu" in prof:  # rocprofv3's MeanOccupancyPerCU of a profiled launch
             occ["measured_mean_waves_per_simd"] = round(prof["mean_occupancy_per_cu"] / 4.0, 3)
         r["occupancy"] = occ
     return r
-
-
-def grid_waves(prog, npaths):
-    """Waves the launch starts.  Per-lane kernel: one per 64 paths, at most one per wave slot
-    (4 SIMDs x the waves per SIMD it was built for, per CU).  Lane-group kernel: four per
-    workgroup of 16 paths (8 paths with 32-lane groups, n > 16), at most two workgroups per CU."""
-    info = prog.kernel_info()
-    if getattr(prog, "layout", "lane") == "group":
-        per_wg = 16 if prog.n <= 16 else 8
-        return 4 * min(-(-npaths // per_wg), 2 * info["cus"])
-    return min(-(-npaths // 64), 4 * info["cus"] * info["waves_per_simd_built"])
 
 
 def host_info():
@@ -366,7 +354,7 @@ def bench_param10(args, out):
                    "launch": launch},
         "roofline": roofline(rl["flops"], rl["kernel_ms"], "param10_learned" + ("" if prog.layout == "lane" else "_group"),
                              kernel="hcg_track_kernel" if prog.layout == "lane" else "hcg_group_kernel",
-                             info=prog.kernel_info(), grid_waves=grid_waves(prog, npaths)),
+                             info=prog.launch_info(npaths, getattr(prog, "blocks_per_cu", 0))),
         "plain_gpu": {"value": round(plain_value, 1), "unit": "paths/s", "kernel_ms": round(rp["kernel_ms"], 3),
                       "steps_per_path": round(rp["steps"] / npaths, 3),
                       "roofline_frac": round(rp["flops"] / (rp["kernel_ms"] * 1e-3) / 1e12 / FP64_PEAK_TFLOPS, 5)},
@@ -423,9 +411,9 @@ def bench_dense(args, out):
     ctx = GpuContext(0)
     opts = make_options()
     if args.layout == "auto":
-        # 3^n paths (81 or 6,561) fill 2 or 103 waves of the per-lane kernel, far fewer than the
-        # GPU's 1,024 SIMDs, or 21 or 1,641 waves of the lane-group kernel (4 paths per wave):
-        # the tuner times both
+        # 3^n paths (81 or 6,561) take 81 or 253 waves of the per-lane kernel (at most one per CU, 1 or 26
+        # lanes of each), far fewer than the GPU's 1,024 SIMDs, or 84 or 1,644 waves of the lane-group
+        # kernel (1 or 4 paths per wave): the tuner times both
         cands = autotune.candidates_for(H.n, lane=((1, 4), (1, 8), (2, 8)), group=(1, 2))
         t0 = time.perf_counter()
         tuned = autotune.tune(ctx, H, S, opts, candidates=cands, force=args.retune)
@@ -447,7 +435,7 @@ def bench_dense(args, out):
                            "launch": launch},
                 "roofline": roofline(r["flops"], r["kernel_ms"], f"dense_n{n}_{npaths}paths" + ("" if prog.layout == "lane" else "_group"),
                                      kernel="hcg_track_kernel" if prog.layout == "lane" else "hcg_group_kernel",
-                                     info=prog.kernel_info(), grid_waves=grid_waves(prog, npaths)),
+                                     info=prog.launch_info(npaths, getattr(prog, "blocks_per_cu", 0))),
                 "steps_per_path": round(r["steps"] / npaths, 3), "solution_counts": counts(rec)})
     if not args.no_cpu:
         sys.path.insert(0, str(REPO))
@@ -534,7 +522,7 @@ def bench_steiner(args, out):
                            "paths": m, "launch": launch},
                 "roofline": roofline(r["flops"], r["kernel_ms"], ("fourbar" if fourbar else "steiner") + f"_{m}paths" + ("" if prog.layout == "lane" else "_group"),
                                      kernel="hcg_track_kernel" if prog.layout == "lane" else "hcg_group_kernel",
-                                     info=prog.kernel_info(), grid_waves=grid_waves(prog, m)),
+                                     info=prog.launch_info(m, getattr(prog, "blocks_per_cu", 0))),
                 "steps_per_path": round(r["steps"] / m, 3), "solution_counts": counts(rec)})
     if not args.no_cpu:
         sys.path.insert(0, str(REPO))
@@ -591,7 +579,7 @@ def bench_mixed(args, out):
                                        "from the host each launch)", "paths": total,
                            "weights": "committed (hcgpu/weights/mixed_step_mlp.npy)"},
                 "roofline": roofline(lfl, lms, "mixed_learned", kernel="hcg_track_multi_kernel",
-                                     info=prog.kernel_info(), grid_waves=grid_waves(prog, total)),
+                                     info=prog.launch_info(total, getattr(prog, "blocks_per_cu", 0))),
                 "plain_gpu": {"value": round(total / pms * 1e3, 1), "unit": "paths/s", "kernel_ms": round(pms, 3)},
                 "learned": {"speedup_vs_plain": round(pms / lms, 3),
                             "steps_per_path": round(sum(int((o.accepted_steps + o.rejected_steps).sum()) for o in louts)

@@ -31,26 +31,28 @@ template <int NN> hipError_t allow_lds32(size_t bytes) {
 
 namespace hcg {
 
-hipError_t group_launch32(int nn, int grid, bool one_per_cu, int lds_per_path, bool mlp_lds, hipStream_t stream,
+hipError_t group_launch32(int nn, int grid, bool wide, int lds_per_path, bool mlp_lds, hipStream_t stream,
                           const hcg_multi_kargs& m, const hcg_gsys* d_sys) {
     const size_t shmem = (mlp_lds ? (size_t)HCG_GROUP_MLP_LDS : 0) + (size_t)(kBlock / GL) * lds_per_path;
     if (nn != 24) return hipErrorInvalidValue;
-    if (one_per_cu) return group_launch32_wide(grid, shmem, lds_per_path, stream, m, d_sys);
+    if (wide) return group_launch32_wide(grid, shmem, lds_per_path, stream, m, d_sys);
     hipError_t e = allow_lds32<24>(shmem);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(hcg_group_kernel32<24>, dim3(grid), dim3(kBlock), shmem, stream, m, d_sys, lds_per_path);
     return hipGetLastError();
 }
 
-hipError_t group_kernel32_blocks_per_cu(int nn, size_t shmem, int* blocks) {
+hipError_t group_kernel32_blocks_per_cu(int nn, bool wide, size_t shmem, int* blocks) {
     if (nn != 24) return hipErrorInvalidValue;
+    if (wide) return group_kernel32_wide_blocks_per_cu(shmem, blocks);
     hipError_t e = allow_lds32<24>(shmem);
     if (e != hipSuccess) return e;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, hcg_group_kernel32<24>, kBlock, shmem);
 }
 
-hipError_t group_kernel32_attributes(int nn, hipFuncAttributes* attr) {
+hipError_t group_kernel32_attributes(int nn, bool wide, hipFuncAttributes* attr) {
     if (nn != 24) return hipErrorInvalidValue;
+    if (wide) return group_kernel32_wide_attributes(attr);
     return hipFuncGetAttributes(attr, reinterpret_cast<const void*>(&hcg_group_kernel32<24>));
 }
 

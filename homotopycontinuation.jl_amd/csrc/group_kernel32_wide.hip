@@ -23,13 +23,27 @@ __global__ void __launch_bounds__(kBlock, 1) hcg_group_kernel32_wide(hcg_multi_k
 
 namespace hcg {
 
+static hipError_t allow_lds(size_t bytes) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&hcg_group_kernel32_wide),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
 hipError_t group_launch32_wide(int grid, size_t shmem, int lds_per_path, hipStream_t stream, const hcg_multi_kargs& m,
                                const hcg_gsys* d_sys) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&hcg_group_kernel32_wide),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+    hipError_t e = allow_lds(shmem);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(hcg_group_kernel32_wide, dim3(grid), dim3(kBlock), shmem, stream, m, d_sys, lds_per_path);
     return hipGetLastError();
+}
+
+hipError_t group_kernel32_wide_blocks_per_cu(size_t shmem, int* blocks) {
+    hipError_t e = allow_lds(shmem);
+    if (e != hipSuccess) return e;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, hcg_group_kernel32_wide, kBlock, shmem);
+}
+
+hipError_t group_kernel32_wide_attributes(hipFuncAttributes* attr) {
+    return hipFuncGetAttributes(attr, reinterpret_cast<const void*>(&hcg_group_kernel32_wide));
 }
 
 }  // namespace hcg

@@ -478,24 +478,22 @@ static int ctx_scalars(hcg_ctx* ctx) {
     return HCG_OK;
 }
 
-// Launch the lane-group kernel: workgroups of four waves, at most blocks_per_cu per CU (default 2),
-// and the groups of each wave that take paths: as few as one wave per SIMD allows, since the groups of a
-// wave wait for each other's evaluations.  All groups of a wave / this rule, measured: n = 15, 64 paths
-// 114.8 / 108.0 ms, 2,048 paths 144.5 / 132.1, 5,000 paths (all groups either way) 166; n = 22, 100 paths
-// 296 / 280, 601 paths 354 / 320.
-static int group_launch(hcg_ctx* ctx, const hcg_program* prog, const hcg_multi_kargs& args, long total,
-                        const hcg_options* opts, hipStream_t stream) {
-    const int waves = hcg::group_block() / 64, most = 64 / hcg::group_lanes_for(prog->group->nn);
-    const int per_cu = opts->blocks_per_cu > 0 ? opts->blocks_per_cu : 2;
-    const long slots = (long)ctx->ncu * waves;
-    const long groups = std::max<long>(1, std::min<long>(most, (total + slots - 1) / slots));
+static hcg::LaunchShape group_shape(const hcg_program* prog, int blocks_per_cu, long total) {
+    return hcg::group_shape(prog->ctx->ncu, hcg::group_block() / 64, 64 / hcg::group_lanes_for(prog->group->nn), blocks_per_cu, total);
+}
+// A launch of 17 to 24 variables with at most one workgroup per CU takes the 512-register instance.
+static bool group_wide(const hcg_program* prog, const hcg::LaunchShape& s) {
+    return hcg::group_lanes_for(prog->group->nn) == 32 && s.workgroups <= prog->ctx->ncu;
+}
+
+static int group_launch(const hcg_program* prog, const hcg_multi_kargs& args, long total, const hcg_options* opts,
+                        hipStream_t stream) {
+    const hcg::LaunchShape s = group_shape(prog, opts->blocks_per_cu, total);
     hcg_multi_kargs m = args;
-    m.sys[0].lanes = (int32_t)groups;
-    long grid = std::min<long>((total + groups * waves - 1) / (groups * waves), (long)ctx->ncu * per_cu);
-    if (grid < 1) grid = 1;
+    m.sys[0].lanes = s.per_wave;
     const bool mlp_lds = opts->learned_step && m.sys[0].mlp;  // the kernel's own staging condition
-    hipError_t e = hcg::group_launch(prog->group->nn, (int)grid, grid <= ctx->ncu, prog->group->lds_per_path, mlp_lds, stream, m,
-                                     prog->group->d_sys);
+    hipError_t e = hcg::group_launch(prog->group->nn, (int)s.workgroups, group_wide(prog, s), prog->group->lds_per_path, mlp_lds,
+                                     stream, m, prog->group->d_sys);
     if (e != hipSuccess) return fail(HCG_ERR_HIP, "group kernel launch: %s", hipGetErrorString(e));
     return HCG_OK;
 }
@@ -519,20 +517,8 @@ static int ctx_launch_state(hcg_ctx* ctx, LaunchState* st) {
     return HCG_OK;
 }
 
-// Grid of the per-lane kernels and the lanes of each wave that take paths.  A batch with fewer than
-// 64 paths per CU is spread over one wave per CU instead of filling 64 lanes of fewer waves: the lanes of
-// a wave wait for each other's branches, and the CUs are free.  More waves than that only touch more
-// lines of private memory (a line holds one dword of 32 lanes) without shortening a path.  Full
-// waves / one wave per CU / four per CU, measured: two-variable parameter homotopy, 2,000 paths 0.29 /
-// 0.21 / 0.29 ms; dense n = 4, 81 paths 6.9 / 5.1 / 5.3; dense n = 8, 400 paths 119.7 / 95.0 / 94.1, 6,561
-// paths 141.8 / 138.3 / 135.7; parameter batch n = 10, 100 paths 43.9 / 35.3 / 37.5, 1,024 paths 49.0 /
-// 47.6 / 61.9, 4,096 paths 43.6 / 45.0 / 59.8.
-static long lane_grid(const hcg_ctx* ctx, const hcg_program* prog, const hcg_options* opts, long npaths, int32_t* lanes) {
-    const int per_cu = opts->blocks_per_cu > 0 ? opts->blocks_per_cu : 4 * prog->waves_per_eu;  // every wave slot of the CU's 4 SIMDs
-    const long slots = (long)ctx->ncu * per_cu;
-    const long waves = std::max<long>(1, std::min(slots, std::max((npaths + 63) / 64, std::min<long>(npaths, ctx->ncu))));
-    *lanes = (int32_t)std::max<long>(1, std::min<long>(64, (npaths + waves - 1) / waves));
-    return std::max<long>(1, std::min<long>(slots, (npaths + *lanes - 1) / *lanes));
+static hcg::LaunchShape lane_shape(const hcg_program* prog, int blocks_per_cu, long npaths) {
+    return hcg::lane_shape(prog->ctx->ncu, prog->waves_per_eu, blocks_per_cu, npaths);
 }
 
 // Enqueue one launch on `stream`: the reset of the launch state (queue head, counters, options)
@@ -579,12 +565,13 @@ static int enqueue_track(hcg_ctx* ctx, const hcg_program* prog, const hcg_batch*
         m.offset[1] = b->npaths;
         m.next_path = st.next;
         m.sys[0] = ka;
-        return group_launch(ctx, prog, m, b->npaths, opts, stream);
+        return group_launch(prog, m, b->npaths, opts, stream);
     }
     const int block = 64;
-    const long grid = lane_grid(ctx, prog, opts, b->npaths, &ka.lanes);
+    const hcg::LaunchShape shape = lane_shape(prog, opts->blocks_per_cu, b->npaths);
+    ka.lanes = shape.per_wave;
     void* args[] = {&ka};
-    HIPCHK(hipModuleLaunchKernel(prog->kernel, (unsigned)grid, 1, 1, block, 1, 1, 0, stream, args, nullptr));
+    HIPCHK(hipModuleLaunchKernel(prog->kernel, (unsigned)shape.workgroups, 1, 1, block, 1, 1, 0, stream, args, nullptr));
     return HCG_OK;
 }
 
@@ -883,15 +870,16 @@ static int hcg_track_multi_impl(hcg_ctx* ctx, const hcg_program* prog, const hcg
         }
     m.offset[S] = (int32_t)total;
     const int block = 64;
-    const long grid = lane_grid(ctx, prog, opts, total, &m.sys[0].lanes);
+    const hcg::LaunchShape shape = lane_shape(prog, opts->blocks_per_cu, total);
+    m.sys[0].lanes = shape.per_wave;
     void* args[] = {&m};
     HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
     if (prog->group) {
         for (int s = 0; s < S; s++) m.sys[s].counters = ctx->d_counters, m.sys[s].opts = ctx->d_opts;
-        rc = group_launch(ctx, prog, m, total, opts, ctx->stream);
+        rc = group_launch(prog, m, total, opts, ctx->stream);
         if (rc) return rc;
     } else {
-        HIPCHK(hipModuleLaunchKernel(prog->kernel, (unsigned)grid, 1, 1, block, 1, 1, 0, ctx->stream, args, nullptr));
+        HIPCHK(hipModuleLaunchKernel(prog->kernel, (unsigned)shape.workgroups, 1, 1, block, 1, 1, 0, ctx->stream, args, nullptr));
     }
     HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
     HIPCHK(hipMemcpyAsync(ctx->last_counters, ctx->d_counters, sizeof(unsigned long long) * 4, hipMemcpyDeviceToHost,
@@ -944,19 +932,18 @@ extern "C" int hcg_group_schedule_info(const hcg_homotopy_desc* const* hs, int32
 // loader reports them), [1] private segment bytes per lane, [2] static LDS bytes per
 // workgroup, [3] waves per SIMD the kernel was built for (lane-group layout: the
 // workgroups that fit on a CU, each one wave per SIMD), [4] workgroup size, [5] CUs.
-extern "C" int hcg_program_kernel_info(const hcg_program* p, int32_t* out6) {
-    if (!p || !out6) return fail(HCG_ERR_INVALID_ARGUMENT, "NULL argument");
+static int kernel_info(const hcg_program* p, bool wide, int32_t* out6) {
     if (p->group) {
         HIPCHK(hipSetDevice(p->ctx->device));
         hipFuncAttributes fa;
-        HIPCHK(hcg::group_kernel_attributes(p->group->nn, &fa));
+        HIPCHK(hcg::group_kernel_attributes(p->group->nn, wide, &fa));
         out6[0] = fa.numRegs;
         out6[1] = (int32_t)fa.localSizeBytes;
         // LDS of a plain launch; the learned step stages its network's weights in front of it
         // (group_mlp_lds_bytes() more per workgroup)
         out6[2] = (hcg::group_block() / hcg::group_lanes_for(p->group->nn)) * p->group->lds_per_path;
         int blocks = 0;  // workgroups per CU; each holds one wave per SIMD
-        HIPCHK(hcg::group_kernel_blocks_per_cu(p->group->nn, (size_t)out6[2], &blocks));
+        HIPCHK(hcg::group_kernel_blocks_per_cu(p->group->nn, wide, (size_t)out6[2], &blocks));
         out6[3] = blocks;
         out6[4] = hcg::group_block();
         out6[5] = p->ctx->ncu;
@@ -970,6 +957,24 @@ extern "C" int hcg_program_kernel_info(const hcg_program* p, int32_t* out6) {
     HIPCHK(hipFuncGetAttribute(&lds, HIP_FUNC_ATTRIBUTE_SHARED_SIZE_BYTES, p->kernel));
     HIPCHK(hipFuncGetAttribute(&maxthr, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, p->kernel));
     out6[0] = regs; out6[1] = priv; out6[2] = lds; out6[3] = p->waves_per_eu; out6[4] = 64; out6[5] = p->ctx->ncu;
+    return HCG_OK;
+}
+extern "C" int hcg_program_kernel_info(const hcg_program* p, int32_t* out6) {
+    if (!p || !out6) return fail(HCG_ERR_INVALID_ARGUMENT, "NULL argument");
+    return kernel_info(p, false, out6);
+}
+
+// The same six for the kernel instance that a launch of npaths paths takes, then [6] its workgroups, [7] the
+// lanes (lane-group layout: groups) of each wave that take paths.
+extern "C" int hcg_launch_info(const hcg_program* p, int64_t npaths, int32_t blocks_per_cu, int32_t* out8) {
+    if (!p || !out8) return fail(HCG_ERR_INVALID_ARGUMENT, "NULL argument");
+    if (npaths < 0 || npaths > INT32_MAX || blocks_per_cu < 0) return fail(HCG_ERR_INVALID_ARGUMENT, "bad path or workgroup count");
+    if (p->certifier) return fail(HCG_ERR_INVALID_ARGUMENT, "not a tracker program");
+    const hcg::LaunchShape s = p->group ? group_shape(p, blocks_per_cu, npaths) : lane_shape(p, blocks_per_cu, npaths);
+    int rc = kernel_info(p, p->group && group_wide(p, s), out8);
+    if (rc) return rc;
+    out8[6] = (int32_t)s.workgroups;
+    out8[7] = s.per_wave;
     return HCG_OK;
 }
 

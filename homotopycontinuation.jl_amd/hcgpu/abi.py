@@ -211,6 +211,7 @@ def lib():
                                P(ctypes.c_long)]
     L.hcg_last_counters.argtypes = [ctypes.c_void_p, P(ctypes.c_uint64)]
     L.hcg_program_kernel_info.argtypes = [ctypes.c_void_p, P(ctypes.c_int32)]
+    L.hcg_launch_info.argtypes = [ctypes.c_void_p, ctypes.c_int64, _I, P(ctypes.c_int32)]
     L.hcg_group_schedule_info.argtypes = [ctypes.c_void_p, ctypes.c_int32, P(ctypes.c_int32)]
     L.hcg_certifier_create.argtypes = [ctypes.c_void_p, P(hcg_system), _I, P(ctypes.c_void_p)]
     L.hcg_certifier_compile_only.argtypes = [P(hcg_system), _I, P(ctypes.c_size_t)]
@@ -240,5 +241,5 @@ HCGPU_SYMBOLS = [
     "hcg_last_counters", "hcg_track_batch_device", "hcg_program_create_multi", "hcg_compile_multi_only",
     "hcg_track_multi", "hcg_program_create_ex", "hcg_compile_ex", "hcg_certifier_create",
     "hcg_certifier_compile_only", "hcg_certify", "hcg_program_kernel_info", "hcg_track_batch_device_noalloc",
-    "hcg_group_schedule_info", "hcg_graph_create", "hcg_graph_launch", "hcg_graph_destroy",
+    "hcg_launch_info", "hcg_group_schedule_info", "hcg_graph_create", "hcg_graph_launch", "hcg_graph_destroy",
 ]

@@ -165,6 +165,9 @@ class Program:
     def kernel_info(self):
         return _kernel_info(self._h)
 
+    def launch_info(self, npaths: int, blocks_per_cu: int = 0):
+        return _launch_info(self._h, npaths, blocks_per_cu)
+
     def close(self):
         if self._h:
             lib().hcg_program_destroy(self._h)
@@ -261,8 +264,22 @@ def _kernel_info(h):
     workgroup size and CUs of a program's tracker kernel (hcg_program_kernel_info)."""
     out = (ctypes.c_int32 * 6)()
     check(lib().hcg_program_kernel_info(h, out))
+    return _kernel_fields(out)
+
+
+def _kernel_fields(out):
     return dict(vgprs=int(out[0]), private_bytes_per_lane=int(out[1]), lds_bytes=int(out[2]),
                 waves_per_simd_built=int(out[3]), workgroup=int(out[4]), cus=int(out[5]))
+
+
+def _launch_info(h, npaths, blocks_per_cu):
+    """kernel_info of the kernel instance that a launch of npaths paths takes, and its waves, workgroups
+    and the lanes (lane-group layout: groups) of each wave that take paths (hcg_launch_info)."""
+    out = (ctypes.c_int32 * 8)()
+    check(lib().hcg_launch_info(h, npaths, blocks_per_cu, out))
+    info = _kernel_fields(out)
+    info.update(workgroups=int(out[6]), waves=int(out[6]) * info["workgroup"] // 64, per_wave=int(out[7]))
+    return info
 
 
 class MultiProgram:
@@ -281,6 +298,9 @@ class MultiProgram:
 
     def kernel_info(self):
         return _kernel_info(self._h)
+
+    def launch_info(self, npaths: int, blocks_per_cu: int = 0):
+        return _launch_info(self._h, npaths, blocks_per_cu)
 
     def close(self):
         if self._h:

@@ -210,6 +210,11 @@ int hcg_last_counters(hcg_ctx* ctx, uint64_t* out4);
  * and the workgroups that fit on a CU with it, each one wave per SIMD),
  * workgroup size, compute units of the device]. */
 int hcg_program_kernel_info(const hcg_program* prog, int32_t* out6);
+/* How a launch of npaths paths runs (blocks_per_cu as in hcg_options): out8 = the six values above
+ * for the kernel instance that it takes (17 to 24 variables in the lane-group layout have a second one
+ * for small batches), then [workgroups, lanes (lane-group layout: groups) of each wave that take
+ * paths]. */
+int hcg_launch_info(const hcg_program* prog, int64_t npaths, int32_t blocks_per_cu, int32_t* out8);
 /* The lane-group layout's slot schedules of nsys homotopies, built and checked against their
  * tapes without a device (no counterpart in the reference; the scheduling evidence of the
  * layout): out[0] = kernel size class (4, 8, 12, 16), out[1] = LDS bytes per path, then per

@@ -264,6 +264,8 @@ hcg_last_counters(ctx, out4) =
     ccall((:hcg_last_counters, libhcgpu), Cint, (Ptr{Cvoid}, Ptr{UInt64}), ctx, out4)
 hcg_program_kernel_info(prog, out6) =
     ccall((:hcg_program_kernel_info, libhcgpu), Cint, (Ptr{Cvoid}, Ptr{Int32}), prog, out6)
+hcg_launch_info(prog, npaths, blocks_per_cu, out8) =
+    ccall((:hcg_launch_info, libhcgpu), Cint, (Ptr{Cvoid}, Int64, Int32, Ptr{Int32}), prog, npaths, blocks_per_cu, out8)
 hcg_group_schedule_info(hs, nsys, out) =
     ccall((:hcg_group_schedule_info, libhcgpu), Cint, (Ptr{Ptr{HcgHomotopyDesc}}, Int32, Ptr{Int32}), hs, nsys, out)
 hcg_generate(h, buf, bufsz, needed, flops6) =

@@ -54,3 +54,15 @@ def test_group_batch_sizes(gpu_ctx, n, npaths):
     np.testing.assert_array_equal(out.code, ref.code[g])
     np.testing.assert_array_equal(out.accepted_steps, ref.accepted_steps[g])
     np.testing.assert_array_equal(out.solution, ref.solution[g])
+
+
+def test_launch_info_follows_the_instance(gpu_ctx):
+    """17 to 24 variables: a launch of at most one workgroup per CU takes the instance with more registers."""
+    F = sparse_param_system(18, 4, 20, seed=18)
+    H = ParameterHomotopy(F, np.zeros(20), [np.zeros(20)], lift_affine=True)
+    p = gpu_ctx.program(H, layout="group")
+    cus = p.kernel_info()["cus"]
+    small, large = p.launch_info(2 * 4 * cus), p.launch_info(2 * 4 * cus + 1)
+    assert (small["workgroups"], large["workgroups"]) == (cus, cus + 1)
+    assert small["vgprs"] > large["vgprs"] and large["vgprs"] == p.kernel_info()["vgprs"]
+    assert (small["waves_per_simd_built"], large["waves_per_simd_built"]) == (1, 2)

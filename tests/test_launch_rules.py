@@ -39,3 +39,30 @@ def test_certify_with_tables(evaluate):
     args = ["{%dL, %dL, %dL, %dL}" % c[2] for c in calls]
     got = evaluate([f"certify_with_tables({c[0]}L, {c[1]}L, CertSplit{a})" for c, a in zip(calls, args)])
     assert got == [c[-1] for c in calls]
+
+
+def _shapes(evaluate, calls):
+    v = evaluate([f"{c}.{f}" for c in calls for f in ("workgroups", "per_wave")])
+    return list(zip(v[::2], v[1::2]))
+
+
+def test_lane_shape(evaluate):
+    """On 256 CUs: one lane of each wave up to one path per CU, full waves from 64 paths per CU on; no more
+    workgroups than wave slots; every path has a lane or waits in the queue of a full grid."""
+    n = [0, 1, 81, 256, 257, 511, 513, 6561, 256 * 63, 256 * 63 + 1, 256 * 64, 256 * 64 + 1, 262144]
+    got = _shapes(evaluate, [f"lane_shape(256, 1, 0, {p}L)" for p in n])
+    assert got == [(1, 1), (1, 1), (81, 1), (256, 1), (129, 2), (256, 2), (171, 3), (253, 26), (256, 63), (253, 64), (256, 64),
+                   (257, 64), (1024, 64)]
+    assert _shapes(evaluate, ["lane_shape(256, 2, 0, 262144L)", "lane_shape(256, 1, 1, 262144L)", "lane_shape(256, 8, 0, 100L)"]) == [
+        (2048, 64), (256, 64), (100, 1)]
+
+
+def test_group_shape(evaluate):
+    """Four 16-lane or two 32-lane groups per wave, four waves per workgroup, 256 CUs."""
+    n = [0, 1, 5, 1024, 1025, 2049, 3073, 8192, 65536]
+    assert _shapes(evaluate, [f"group_shape(256, 4, 4, 0, {p}L)" for p in n]) == [
+        (1, 1), (1, 1), (2, 1), (256, 1), (129, 2), (171, 3), (193, 4), (512, 4), (512, 4)]
+    n = [601, 1024, 1025, 2048, 2049, 4096, 4097, 8192]
+    assert _shapes(evaluate, [f"group_shape(256, 4, 2, 0, {p}L)" for p in n]) == [
+        (151, 1), (256, 1), (129, 2), (256, 2), (257, 2), (512, 2), (512, 2), (512, 2)]
+    assert _shapes(evaluate, ["group_shape(256, 4, 4, 1, 65536L)"]) == [(256, 4)]
