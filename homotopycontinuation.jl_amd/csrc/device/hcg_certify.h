@@ -225,7 +225,7 @@ __device__ __noinline__ void cert_refine_dd(cdd* xd, const cplx* C, const double
 #if HCG_CERT_NCE > 0
 // A candidate's time is the latency of its interpreted evaluations (registers in private memory), so what
 // does not depend on the candidate is taken out of them: 16,000 candidates of the n = 10 parameter
-// system on 16 parameter vectors 47.2 -> 8.0 ms for the whole call.
+// system on 16 parameter vectors 46.9 -> 7.0 ms for the whole call.
 // Coefficient tables of one parameter vector, in doubles from its start: double-double values, boxes and
 // balls of the evaluation's coefficients, then boxes and balls of the Jacobian's.
 #define CERT_IE (4 * HCG_CERT_NCE)

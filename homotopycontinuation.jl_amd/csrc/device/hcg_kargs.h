@@ -12,7 +12,7 @@ typedef struct hcg_kargs {
     int32_t npaths;
     int32_t log_capacity;
     int32_t ngroups;
-    int32_t lanes;                 // lanes of each wave that track paths (per-lane kernels)
+    int32_t lanes;                 // lanes (lane-group kernels: groups) of each wave that take paths
     const double* starts;          // npaths * n complex
     double t1, t0;
     const double* start_params;    // nparams complex (PARAMETER)

@@ -26,8 +26,8 @@ enum { NEWT_CONVERGED = 0, NEWT_TERMINATED, NEWT_MAX_ITERS, NEWT_SINGULARITY };
 
 struct NewtRes { int code; double accuracy; int iters; double omega, theta, mu_low, norm_dx0; };
 
-// End-of-path work left for lane_close: the rest of the step that reached the end of the
-// segment (PEND_STEP), then tracking_stopped! (PEND_STOP).
+// End-of-path work left for the wave's refill: the rest of the step that reached the end of the
+// segment (PEND_STEP, done by one more lane_iter), then tracking_stopped! (PEND_STOP, in lane_close).
 enum { PEND_NONE = 0, PEND_STEP, PEND_STOP };
 
 struct Lane {
@@ -87,7 +87,7 @@ struct Lane {
     const unsigned short* mlp_w;  // BF16 weights in LDS, or null (plain rule only)
     double flops;  // counted FP64 flops of this path
     int guard;     // loop iterations of the current path (each performs >= 1 tracker step)
-    // work at the end of a path that waits for the wave's next refill (lane_close)
+    // work at the end of a path that waits for the wave's next refill
     int pend;
     double pend_ds0;
     NewtRes pend_res;
@@ -1389,7 +1389,8 @@ __device__ __noinline__ void log_step(Lane& L, const NewtRes& res, int acc) {
 // step!(tracker), src/tracker.jl:851-926; returns !last_step_failed.  The step that ends the path
 // (outside the singular endgame) returns with L.pend = PEND_STEP after its Newton correction, and
 // the next call does the rest: refinement in double-double and the predictor's update, several
-// ordinary evaluations' work, which lane_close runs for all ended lanes of a wave at once.
+// ordinary evaluations' work, which all ended lanes of a wave do together, in the lane_iter at the
+// wave's refill (before lane_close).
 __device__ __forceinline__ int tracker_step(Lane& L) {
     const hcg_options* o = L.o;
     NewtRes res;
@@ -1799,7 +1800,7 @@ __device__ __noinline__ void eg_step(Lane& L) {
         singular_post(L, max_steps);
         return;
     }
-    if (L.pend == PEND_STEP) return;  // the path has reached its end: continued by lane_close
+    if (L.pend == PEND_STEP) return;  // the path has reached its end: continued by lane_iter at the wave's refill
     L.eg_code = tc_to_eg(L.code);
     if (L.eg_code != EG_TRACKING) { L.pend = PEND_STOP; return; }  // tracking_stopped!, in lane_close
     L.jtzf0 = L.jtzf1; L.jtzf1 = jump;

@@ -294,9 +294,14 @@ static int hcg_generate_impl(const hcg_homotopy_desc* h, char* buf, size_t bufsz
 // solve's matrix stays in the 512 registers of one wave per SIMD, and a loaded kernel waits for the traffic
 // of its lanes' private state, which a second wave doubles.  One against two waves, measured: parameter
 // batch n = 10, 1,024 paths plain 48.5 / 50.5 ms, 61,777 plain 153.7 / 163.7, 262,144 learned 294.6 /
-// 307.8; dense n = 8, 6,561 paths 152.6 / 251.2.  Past n = 10 the matrix does not fit and the long
-// straight-line evaluations need a second wave to issue beside: shared-factor cubics n = 12, learned, 30,000
-// paths 317.7 / 341.4 ms, 131,072 paths 739.8 / 640.7, 531,441 paths 2,314.9 / 1,907.1.
+// 307.8; dense n = 8, 6,561 paths 152.6 / 251.2; sparse quadrics, 65,536 paths plain: n = 9 69.1 / 154.9,
+// n = 8 44.4 / 52.3, n = 6 20.6 / 22.9, n = 4 7.9 / 8.4, n = 3 4.7 / 5.1; two variables, 65,536 paths 1.03 / 1.08.
+// Only two-variable batches that fill every wave many times are faster with two: 262,144 paths 2.38 / 2.23,
+// 1,048,576 paths 8.0 / 7.2.  Past n = 10 the matrix does not fit and the long straight-line evaluations need
+// a second wave to issue beside: shared-factor cubics n = 12, learned, 131,072 paths 739.8 / 640.7, 531,441
+// paths 2,314.9 / 1,907.1, but 30,000 paths 317.7 / 341.4 (the instance is fixed when the program is
+// made, before the batch is known).  Past n = 12 the lane-group layout is the host's default; per-lane
+// programs of that size keep two.
 static int default_waves(const hcg_homotopy_desc* const* hs, int32_t nsys) {
     int n = 0;
     for (int s = 0; s < nsys; s++) n = std::max<int>(n, hs[s]->n);

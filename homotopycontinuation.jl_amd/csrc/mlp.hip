@@ -8,7 +8,8 @@
 // mlp_tile: one workgroup of four waves takes tiles of 32 records through forward and backward.  The
 // products over the hidden layers run on the FP32 matrix cores (v_mfma_f32_16x16x4: FP32
 // operands and sums, so no precision is given up for them), activations and weights staged in
-// LDS with rows of 68 floats, which the 16 x 4 operand reads cross without bank conflicts.  GELU and
+// LDS with rows of 68 floats, which the operand reads along rows cross without bank conflicts (the transposed
+// ones, of da2, h1 and w2 in the backward products, put up to four addresses on a bank).  GELU and
 // its derivative are computed once per activation, the derivative kept in the registers of the
 // lane that needs it.  Each workgroup writes its partial gradient; grad_step adds the partials in a
 // fixed order and, in training, makes the Adam step in the same launch.  A batch of 4,096 is 128
