@@ -1,6 +1,6 @@
 """Small batches of the lane-group layout: path counts at which the groups of a wave that take paths,
-or the kernel instance, change; against the oracle.  Per-lane layout: spread over one wave per CU,
-path counts around the points where the lanes of a wave
+or the kernel instance, change; against the oracle.  Per-lane layout: spread over up to one wave per
+CU, path counts around the points where the lanes of a wave
 that take paths change (1 up to one path per CU, 64 from 64 paths per CU on)."""
 import numpy as np
 import pytest
